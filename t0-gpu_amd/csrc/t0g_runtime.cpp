@@ -314,8 +314,8 @@ static uint32_t sk_grid(const GemmPlan &p, uint32_t num_cus) {
 //     or the stage's first k row (M/N-contiguous) and cut to 2 GiB; the offsets
 //     used from there stay below 2 GiB for leading dimensions below these bounds
 //     (256 rows of a K-contiguous tile; 64 k rows plus one row of a stage).
-//   Elementwise: everything else (_u kernels, 32-bit element offsets).
-enum class OperandPath { Fast, Wide, Elementwise };
+//   Staged: everything else (_u kernels, 32-bit byte offsets).
+enum class OperandPath { Fast, Wide, Staged };
 constexpr uint32_t kMaxKMajorLd = 1u << 22;
 constexpr uint32_t kMaxMnMajorLd = (1u << 24) - 256;
 
@@ -332,16 +332,16 @@ static bool ld_fits_256(uint32_t t, uint32_t lda, uint32_t ldb) {
 
 static OperandPath operand_path(uint64_t a, uint64_t b, uint32_t m, uint32_t n, uint32_t k, uint32_t lda,
                                 uint32_t ldb, uint32_t t) {
-    if ((a & 15) || (b & 15) || (lda & 7) || (ldb & 7)) return OperandPath::Elementwise;
-    if (a_k_major(t) ? (k & 7) != 0 : ((m & 7) != 0 || m < 8)) return OperandPath::Elementwise;
-    if (b_k_major(t) ? (k & 7) != 0 : ((n & 7) != 0 || n < 8)) return OperandPath::Elementwise;
+    if ((a & 15) || (b & 15) || (lda & 7) || (ldb & 7)) return OperandPath::Staged;
+    if (a_k_major(t) ? (k & 7) != 0 : ((m & 7) != 0 || m < 8)) return OperandPath::Staged;
+    if (b_k_major(t) ? (k & 7) != 0 : ((n & 7) != 0 || n < 8)) return OperandPath::Staged;
     const uint64_t a_elems = a_k_major(t) ? (uint64_t)m * lda : (uint64_t)k * lda;
     const uint64_t b_elems = b_k_major(t) ? (uint64_t)n * ldb : (uint64_t)k * ldb;
     if (a_elems < (1ull << 30) && b_elems < (1ull << 30)) return OperandPath::Fast;
     if (lda < (a_k_major(t) ? kMaxKMajorLd : kMaxMnMajorLd) && ldb < (b_k_major(t) ? kMaxKMajorLd : kMaxMnMajorLd) &&
         ld_fits_256(t, lda, ldb))
         return OperandPath::Wide;
-    return OperandPath::Elementwise;
+    return OperandPath::Staged;
 }
 
 // allow_fused: the caller can run the in-kernel split-K reduction (its sync
@@ -354,10 +354,10 @@ static OperandPath operand_path(uint64_t a, uint64_t b, uint32_t m, uint32_t n, 
 static int make_plan(const TileDef *tile, uint32_t transpose, bool out_bf16, OperandPath path, bool fits_256,
                      uint32_t m, uint32_t n, uint32_t k, uint32_t split_req, GemmPlan *p, bool allow_fused = false,
                      bool exact_split = false) {
-    const bool aligned = path != OperandPath::Elementwise, wide = path == OperandPath::Wide;
+    const bool aligned = path != OperandPath::Staged, wide = path == OperandPath::Wide;
     bool stream_k = split_req == T0G_STREAM_K;
     if (stream_k) split_req = 1;
-    if (!aligned && tile->bm == 256) tile = &kTiles[1];   // no element-wise-load variant of the 256x256 tile
+    if (!aligned && tile->bm == 256) tile = &kTiles[1];   // no staged variant of the 256x256 tile
     if (!fits_256 && tile->bm == 256) tile = &kTiles[1];
     if (wide) tile = &kTiles[0];                           // the wide kernels are 256x256 only
     if (tile->bm != 256 || k == 0 || wide) stream_k = false;   // the data-parallel kernel then
@@ -427,12 +427,12 @@ static int make_plan(const TileDef *tile, uint32_t transpose, bool out_bf16, Ope
     return T0G_OK;
 }
 
-// The element-wise kernels (operands the fast path cannot take) use 32-bit
-// element offsets.
+// The staged kernels (operands the fast path cannot take) use 32-bit byte
+// offsets.
 static int check_extent(const char *what, uint64_t rows, uint64_t ld) {
     if (rows * ld >= (1ull << 31))
         return fail(T0G_ERR_INVALID_ARG,
-                    "%s spans %llu elements; unaligned operands (taken element-wise) must stay below 2^31", what,
+                    "%s spans %llu elements; unaligned operands must stay below 2^31", what,
                     (unsigned long long)(rows * ld));
     return T0G_OK;
 }
@@ -660,7 +660,7 @@ static int resolve_desc(const t0g_gemm_desc *d, t0g_gemm_config *cfg, GemmPlan *
         return fail(T0G_ERR_UNSUPPORTED_CONFIG, "split_k=%u > %u", sk, kMaxSplitK);
     const TileDef *tile = plan_tile(cfg, d->m, d->k, d->n, sk);
     const OperandPath path = operand_path(d->a, d->b, d->m, d->n, d->k, o->lda, o->ldb, t);
-    if (path == OperandPath::Elementwise) {
+    if (path == OperandPath::Staged) {
         if ((rc = check_extent("A", a_k_major(t) ? d->m : d->k, o->lda))) return rc;
         if ((rc = check_extent("B", b_k_major(t) ? d->n : d->k, o->ldb))) return rc;
     }
@@ -1225,7 +1225,7 @@ static int dispatch_ref(t0g_device *dev, const t0g_kernel *kn, uint32_t tiles_m,
         const TileDef *tile = plan_tile(&cfg, o.m, o.k, o.n, sk);
         const OperandPath path = operand_path(o.a, o.b, o.m, o.n, o.k, o.lda, o.ldb, cfg.transpose);
         int rc;
-        if (path == OperandPath::Elementwise) {
+        if (path == OperandPath::Staged) {
             if ((rc = check_extent("X", o.m, o.lda))) return rc;
             if ((rc = check_extent("WT", cfg.transpose == T0G_NN ? o.k : o.n, o.ldb))) return rc;
         }
@@ -1334,7 +1334,7 @@ static int dispatch_gemm(t0g_device *dev, const t0g_kernel *kn, const uint32_t g
     int rc;
     const TileDef *tile = find_tile(cfg.tile_m, cfg.tile_n, cfg.tile_k, cfg.wg_size);
     const OperandPath path = operand_path(o.a, o.b, o.m, o.n, o.k, o.lda, o.ldb, cfg.transpose);
-    if (path == OperandPath::Elementwise) {
+    if (path == OperandPath::Staged) {
         if ((rc = check_extent("X", o.m, o.lda))) return rc;
         if ((rc = check_extent("WT", cfg.transpose == T0G_NN ? o.k : o.n, o.ldb))) return rc;
     }
