@@ -861,25 +861,28 @@ __device__ __forceinline__ void mfma_rows(f32x16_t (&acc)[SM][SN], const bf16x8_
 // stage's DMA instructions are spread evenly over its steps.  BK 64 makes each
 // K-contiguous LDS row a whole 128-byte line, so every DMA request fetches
 // complete cache lines (the deep-ring kernels, one workgroup per CU).
-template <bool CHECK, uint32_t BK, int NS, uint32_t A_BYTES, uint32_t STAGE, int kVmemPerStage, int SM, int SN,
+template <bool CHECK, bool OWN, uint32_t BK, int NS, uint32_t A_BYTES, uint32_t STAGE, int kVmemPerStage, int SM, int SN,
           class OpA, class OpB>
 __device__ __forceinline__ void k_pipeline(f32x16_t (&acc)[SM][SN], const OpA& la, const OpB& lb, const T0gGemmArgs& p,
                                            uint32_t a_bytes, uint32_t b_bytes, uint32_t kbeg, uint32_t kend, int nst,
                                            uint32_t lds0) {
-    static_assert((BK == 32 || BK == 64) && NS >= 4, "ring of BK 32 or 64 stages");
+    static_assert((BK == 32 || BK == 64) && NS >= (OWN ? 4 : 3), "ring of BK 32 or 64 stages");
     constexpr int kSteps = (int)BK / 16;
     // DMA instructions of the stage before K step i: [kD(i), kD(i + 1))
-    constexpr int kPer = (kVmemPerStage + kSteps - 1) / kSteps;
-#define T0G_KD(i) ((i) * kPer < kVmemPerStage ? (i) * kPer : kVmemPerStage)
+    constexpr int kDma = OWN ? kVmemPerStage : 0;
+    constexpr int kPer = (kDma + kSteps - 1) / kSteps;
+#define T0G_KD(i) ((i) * kPer < kDma ? (i) * kPer : kDma)
     bf16x8_t fa0[SM], fb0[SN], fa1[SM], fb1[SN];
     {
         // Prologue: stages 0 .. NS-2 in flight; stages 0 and 1 must have landed.
+        if constexpr (OWN) {
 #pragma unroll
-        for (int s = 0; s < NS - 1; ++s) {
-            la.template issue<CHECK>(lds0 + s * STAGE, p.a, a_bytes, p.lda, kbeg + s * BK, kend);
-            lb.template issue<CHECK>(lds0 + s * STAGE + A_BYTES, p.b, b_bytes, p.ldb, kbeg + s * BK, kend);
+            for (int s = 0; s < NS - 1; ++s) {
+                la.template issue<CHECK>(lds0 + s * STAGE, p.a, a_bytes, p.lda, kbeg + s * BK, kend);
+                lb.template issue<CHECK>(lds0 + s * STAGE + A_BYTES, p.b, b_bytes, p.ldb, kbeg + s * BK, kend);
+            }
+            T0G_WAIT_VMCNT(kVmemPerStage * (NS - 3));
         }
-        T0G_WAIT_VMCNT(kVmemPerStage * (NS - 3));
         barrier_no_fence();
         la.template read<0>(lds0, fa0);
         lb.template read<0>(lds0 + A_BYTES, fb0);
@@ -889,8 +892,11 @@ __device__ __forceinline__ void k_pipeline(f32x16_t (&acc)[SM][SN], const OpA& l
         for (int s = 0; s < nst; ++s) {
             const uint32_t nxt = cur + STAGE == NS * STAGE ? 0 : cur + STAGE;
             const uint32_t kf = kbeg + (uint32_t)(s + NS - 1) * BK;
-            const u32x4_t ra = la.rsrc(p.a, a_bytes, p.lda, kf);
-            const u32x4_t rb = lb.rsrc(p.b, b_bytes, p.ldb, kf);
+            u32x4_t ra{}, rb{};
+            if constexpr (OWN) {
+                ra = la.rsrc(p.a, a_bytes, p.lda, kf);
+                rb = lb.rsrc(p.b, b_bytes, p.ldb, kf);
+            }
             // K step i of stage s reads step i + 1's fragments (the last step:
             // step 0 of stage s + 1, landed before the last barrier).
             mfma_rows<0, kSteps, T0G_KD(0), T0G_KD(1) - T0G_KD(0), CHECK>(
@@ -903,7 +909,7 @@ __device__ __forceinline__ void k_pipeline(f32x16_t (&acc)[SM][SN], const OpA& l
                 mfma_rows<3, kSteps, T0G_KD(3), T0G_KD(4) - T0G_KD(3), CHECK>(
                     acc, fa1, fb1, fa0, fb0, la, lb, lds0 + cur, lds0 + nxt, lds0 + fill, ra, rb, kf, kend);
             }
-            T0G_WAIT_VMCNT(kVmemPerStage * (NS - 3));   // stage s+2 has landed
+            if constexpr (OWN) T0G_WAIT_VMCNT(kVmemPerStage * (NS - 3));   // stage s+2 has landed
             barrier_no_fence();
             fill = cur;
             cur = nxt;
@@ -971,40 +977,46 @@ __device__ __forceinline__ void mfma_step_dma(f32x16_t (&acc)[SM][SN], const bf1
 // One stage: read stage `nxt` into (na, nb), multiply the current stage from
 // (fa, fb), refill `fill` with stage kf's DMA, then wait for the stage two
 // ahead and meet at the barrier.
-template <bool CHECK, int NS, uint32_t STAGE, int kVmemPerStage, int SM, int SN, class OpA, class OpB>
-__device__ __forceinline__ void deep_stage(f32x16_t (&acc)[SM][SN], const bf16x8_t (&fa)[4][SM],
+template <bool CHECK, bool OWN, int NS, uint32_t STAGE, int kVmemPerStage, int NACC, int SM, int SN, class OpA, class OpB>
+__device__ __forceinline__ void deep_stage(f32x16_t (&acc)[NACC][SM][SN], const bf16x8_t (&fa)[4][SM],
                                            const bf16x8_t (&fb)[4][SN], bf16x8_t (&na)[4][SM], bf16x8_t (&nb)[4][SN],
                                            const OpA& la, const OpB& lb, const T0gGemmArgs& p, uint32_t a_bytes,
                                            uint32_t b_bytes, uint32_t nxt, uint32_t fill, uint32_t kf, uint32_t kend) {
-    constexpr int kPer = (kVmemPerStage + 3) / 4;
-#define T0G_KD4(i) ((i) * kPer < kVmemPerStage ? (i) * kPer : kVmemPerStage)
+    constexpr int kDma = OWN ? kVmemPerStage : 0;
+    constexpr int kPer = (kDma + 3) / 4;
+#define T0G_KD4(i) ((i) * kPer < kDma ? (i) * kPer : kDma)
     read_stage4(la, lb, nxt, na, nb);
-    const u32x4_t ra = la.rsrc(p.a, a_bytes, p.lda, kf);
-    const u32x4_t rb = lb.rsrc(p.b, b_bytes, p.ldb, kf);
-    mfma_step_dma<T0G_KD4(0), T0G_KD4(1) - T0G_KD4(0), CHECK>(acc, fa[0], fb[0], la, lb, fill, ra, rb, kf, kend);
-    mfma_step_dma<T0G_KD4(1), T0G_KD4(2) - T0G_KD4(1), CHECK>(acc, fa[1], fb[1], la, lb, fill, ra, rb, kf, kend);
-    mfma_step_dma<T0G_KD4(2), T0G_KD4(3) - T0G_KD4(2), CHECK>(acc, fa[2], fb[2], la, lb, fill, ra, rb, kf, kend);
-    mfma_step_dma<T0G_KD4(3), T0G_KD4(4) - T0G_KD4(3), CHECK>(acc, fa[3], fb[3], la, lb, fill, ra, rb, kf, kend);
+    u32x4_t ra{}, rb{};
+    if constexpr (OWN) {
+        ra = la.rsrc(p.a, a_bytes, p.lda, kf);
+        rb = lb.rsrc(p.b, b_bytes, p.ldb, kf);
+    }
+    mfma_step_dma<T0G_KD4(0), T0G_KD4(1) - T0G_KD4(0), CHECK>(acc[0 % NACC], fa[0], fb[0], la, lb, fill, ra, rb, kf, kend);
+    mfma_step_dma<T0G_KD4(1), T0G_KD4(2) - T0G_KD4(1), CHECK>(acc[1 % NACC], fa[1], fb[1], la, lb, fill, ra, rb, kf, kend);
+    mfma_step_dma<T0G_KD4(2), T0G_KD4(3) - T0G_KD4(2), CHECK>(acc[2 % NACC], fa[2], fb[2], la, lb, fill, ra, rb, kf, kend);
+    mfma_step_dma<T0G_KD4(3), T0G_KD4(4) - T0G_KD4(3), CHECK>(acc[3 % NACC], fa[3], fb[3], la, lb, fill, ra, rb, kf, kend);
 #undef T0G_KD4
-    T0G_WAIT_VMCNT(kVmemPerStage * (NS - 3));   // the stage two ahead has landed
+    if constexpr (OWN) T0G_WAIT_VMCNT(kVmemPerStage * (NS - 3));   // the stage two ahead has landed
     barrier_no_fence();
 }
 
-template <bool CHECK, int NS, uint32_t A_BYTES, uint32_t STAGE, int kVmemPerStage, int SM, int SN, class OpA,
-          class OpB>
-__device__ __forceinline__ void k_pipeline_deep(f32x16_t (&acc)[SM][SN], const OpA& la, const OpB& lb,
+template <bool CHECK, bool OWN, int NS, uint32_t A_BYTES, uint32_t STAGE, int kVmemPerStage, int NACC, int SM, int SN,
+          class OpA, class OpB>
+__device__ __forceinline__ void k_pipeline_deep(f32x16_t (&acc)[NACC][SM][SN], const OpA& la, const OpB& lb,
                                                 const T0gGemmArgs& p, uint32_t a_bytes, uint32_t b_bytes,
                                                 uint32_t kbeg, uint32_t kend, int nst, uint32_t lds0) {
-    static_assert(NS >= 4, "ring of at least 4 stages");
+    static_assert(NS >= (OWN ? 4 : 3), "ring of at least 4 stages");
     constexpr uint32_t BK = 64;
     bf16x8_t fa0[4][SM], fb0[4][SN], fa1[4][SM], fb1[4][SN];
     // Prologue: stages 0 .. NS-2 in flight; stages 0 and 1 must have landed.
+    if constexpr (OWN) {
 #pragma unroll
-    for (int s = 0; s < NS - 1; ++s) {
-        la.template issue<CHECK>(lds0 + s * STAGE, p.a, a_bytes, p.lda, kbeg + s * BK, kend);
-        lb.template issue<CHECK>(lds0 + s * STAGE + A_BYTES, p.b, b_bytes, p.ldb, kbeg + s * BK, kend);
+        for (int s = 0; s < NS - 1; ++s) {
+            la.template issue<CHECK>(lds0 + s * STAGE, p.a, a_bytes, p.lda, kbeg + s * BK, kend);
+            lb.template issue<CHECK>(lds0 + s * STAGE + A_BYTES, p.b, b_bytes, p.ldb, kbeg + s * BK, kend);
+        }
+        T0G_WAIT_VMCNT(kVmemPerStage * (NS - 3));
     }
-    T0G_WAIT_VMCNT(kVmemPerStage * (NS - 3));
     barrier_no_fence();
     read_stage4(la, lb, lds0, fa0, fb0);
 
@@ -1014,7 +1026,7 @@ __device__ __forceinline__ void k_pipeline_deep(f32x16_t (&acc)[SM][SN], const O
         {
             const uint32_t nxt = cur + STAGE == NS * STAGE ? 0 : cur + STAGE;
             const uint32_t kf = kbeg + (uint32_t)(s + NS - 1) * BK;
-            deep_stage<CHECK, NS, STAGE, kVmemPerStage>(acc, fa0, fb0, fa1, fb1, la, lb, p, a_bytes, b_bytes,
+            deep_stage<CHECK, OWN, NS, STAGE, kVmemPerStage>(acc, fa0, fb0, fa1, fb1, la, lb, p, a_bytes, b_bytes,
                                                         lds0 + nxt, lds0 + fill, kf, kend);
             fill = cur;
             cur = nxt;
@@ -1022,7 +1034,7 @@ __device__ __forceinline__ void k_pipeline_deep(f32x16_t (&acc)[SM][SN], const O
         if (s + 1 < nst) {
             const uint32_t nxt = cur + STAGE == NS * STAGE ? 0 : cur + STAGE;
             const uint32_t kf = kbeg + (uint32_t)(s + NS) * BK;
-            deep_stage<CHECK, NS, STAGE, kVmemPerStage>(acc, fa1, fb1, fa0, fb0, la, lb, p, a_bytes, b_bytes,
+            deep_stage<CHECK, OWN, NS, STAGE, kVmemPerStage>(acc, fa1, fb1, fa0, fb0, la, lb, p, a_bytes, b_bytes,
                                                         lds0 + nxt, lds0 + fill, kf, kend);
             fill = cur;
             cur = nxt;
@@ -1227,18 +1239,19 @@ __device__ __forceinline__ void gemm_tile_fast(const T0gGemmArgs& p, const T0gGe
                 k_pipeline_ksplit<true, NS, A_BYTES, STAGE, kVmemPerStage>(acc4, ka, kb, p, a_bytes, b_bytes, kbeg,
                                                                            kend, nst, lds0);
         } else if constexpr (BK == 64 && SM * SN == 1) {
+            f32x16_t(&accd)[1][SM][SN] = *reinterpret_cast<f32x16_t(*)[1][SM][SN]>(&acc);
             if ((kend - kbeg) % BK == 0)
-                k_pipeline_deep<false, NS, A_BYTES, STAGE, kVmemPerStage>(acc, la, lb, p, a_bytes, b_bytes, kbeg,
+                k_pipeline_deep<false, true, NS, A_BYTES, STAGE, kVmemPerStage>(accd, la, lb, p, a_bytes, b_bytes, kbeg,
                                                                           kend, nst, lds0);
             else
-                k_pipeline_deep<true, NS, A_BYTES, STAGE, kVmemPerStage>(acc, la, lb, p, a_bytes, b_bytes, kbeg,
+                k_pipeline_deep<true, true, NS, A_BYTES, STAGE, kVmemPerStage>(accd, la, lb, p, a_bytes, b_bytes, kbeg,
                                                                          kend, nst, lds0);
         } else {
             if ((kend - kbeg) % BK == 0)
-                k_pipeline<false, BK, NS, A_BYTES, STAGE, kVmemPerStage>(acc, la, lb, p, a_bytes, b_bytes, kbeg,
+                k_pipeline<false, true, BK, NS, A_BYTES, STAGE, kVmemPerStage>(acc, la, lb, p, a_bytes, b_bytes, kbeg,
                                                                           kend, nst, lds0);
             else
-                k_pipeline<true, BK, NS, A_BYTES, STAGE, kVmemPerStage>(acc, la, lb, p, a_bytes, b_bytes, kbeg,
+                k_pipeline<true, true, BK, NS, A_BYTES, STAGE, kVmemPerStage>(acc, la, lb, p, a_bytes, b_bytes, kbeg,
                                                                          kend, nst, lds0);
         }
     }
@@ -1426,7 +1439,8 @@ __device__ __forceinline__ uint32_t bf16_bits_ref(float x) {
 // a grid of 8192 workgroups: 64 Mi elements in 58.4 against 66.6 us; a full grid
 // of that form took 62.4 us, and more loads in flight per lane were slower.
 // Whole waves run without per-lane bounds tests (those cost 61.2 us).
-extern "C" __global__ void __launch_bounds__(256) t0g_f32_to_bf16_rne(T0gConvertArgs p) {
+namespace t0g {
+__device__ __forceinline__ void convert_f32(const T0gConvertArgs& p, uint32_t block) {
     typedef float f32x4_t __attribute__((ext_vector_type(4)));
     typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
     typedef const __attribute__((address_space(1))) f32x4_t gf32x4_t;
@@ -1439,10 +1453,10 @@ extern "C" __global__ void __launch_bounds__(256) t0g_f32_to_bf16_rne(T0gConvert
         gf32x4_t* const s = reinterpret_cast<gf32x4_t*>((uintptr_t)p.src);
         gu32x2_t* const d = reinterpret_cast<gu32x2_t*>((uintptr_t)p.dst);
         auto pack4 = [](f32x4_t v) {
-            return u32x2_t{t0g::bf16_bits_ref(v[0]) | (t0g::bf16_bits_ref(v[1]) << 16),
-                           t0g::bf16_bits_ref(v[2]) | (t0g::bf16_bits_ref(v[3]) << 16)};
+            return u32x2_t{bf16_bits_ref(v[0]) | (bf16_bits_ref(v[1]) << 16),
+                           bf16_bits_ref(v[2]) | (bf16_bits_ref(v[3]) << 16)};
         };
-        for (uint64_t wb = ((uint64_t)blockIdx.x * 4 + wave) * 128; wb < n4; wb += step) {
+        for (uint64_t wb = ((uint64_t)block * 4 + wave) * 128; wb < n4; wb += step) {
             if (wb + 128 <= n4) {
                 const f32x4_t a = __builtin_nontemporal_load(s + wb + lane);
                 const f32x4_t b = __builtin_nontemporal_load(s + wb + 64 + lane);
@@ -1457,9 +1471,21 @@ extern "C" __global__ void __launch_bounds__(256) t0g_f32_to_bf16_rne(T0gConvert
         return;
     }
     const uint64_t stride = (uint64_t)p.grid_blocks * 256;
-    for (uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x; i < p.n; i += stride)
+    for (uint64_t i = (uint64_t)block * 256 + threadIdx.x; i < p.n; i += stride)
         reinterpret_cast<__attribute__((address_space(1))) uint16_t*>((uintptr_t)p.dst)[i] =
-            (uint16_t)t0g::bf16_bits_ref(reinterpret_cast<const __attribute__((address_space(1))) float*>((uintptr_t)p.src)[i]);
+            (uint16_t)bf16_bits_ref(reinterpret_cast<const __attribute__((address_space(1))) float*>((uintptr_t)p.src)[i]);
+}
+}  // namespace t0g
+
+extern "C" __global__ void __launch_bounds__(256) t0g_f32_to_bf16_rne(T0gConvertArgs p) {
+    t0g::convert_f32(p, blockIdx.x);
+}
+// Two tensors in one launch: the first p.a.grid_blocks workgroups take p.a.
+extern "C" __global__ void __launch_bounds__(256) t0g_f32_to_bf16_rne_pair(T0gConvertPairArgs p) {
+    if (blockIdx.x < p.a.grid_blocks)
+        t0g::convert_f32(p.a, blockIdx.x);
+    else
+        t0g::convert_f32(p.b, blockIdx.x - p.a.grid_blocks);
 }
 
 // ---------------------------------------------------------------------------
@@ -1474,31 +1500,47 @@ extern "C" __global__ void __launch_bounds__(256) t0g_f32_to_bf16_rne(T0gConvert
 #define T0G_WPE_64x64 1, 4
 #define T0G_PIPE_128x128 32, 4
 #define T0G_PIPE_64x64 32, 4
-// stages in flight in VGPRs (_u)
-#define T0G_STAGED_128x128 2
-#define T0G_STAGED_64x64 4
-#define T0G_GEMM(NAME, BM, BN, WM, WN, AK, BKM, OBF, AL)                                       \
+#define T0G_GEMM(NAME, BM, BN, WM, WN, AK, BKM, OBF)                                           \
     extern "C" __global__ void __launch_bounds__(64 * WM * WN)                                   \
         __attribute__((amdgpu_waves_per_eu(T0G_WPE_##BM##x##BN))) NAME(T0gGemmArgs p) {          \
-        if constexpr (AL)                                                                        \
-            t0g::gemm_tile_fast<BM, BN, WM, WN, AK, BKM, OBF, T0G_PIPE_##BM##x##BN>(p);            \
-        else                                                                                     \
-            t0g::gemm_tile_staged<BM, BN, WM, WN, AK, BKM, OBF, T0G_STAGED_##BM##x##BN>(p);                                 \
+        t0g::gemm_tile_fast<BM, BN, WM, WN, AK, BKM, OBF, T0G_PIPE_##BM##x##BN>(p);              \
     }
 
-#define T0G_GEMM_LAYOUTS(PFX, BM, BN, WM, WN, OUTN, OBF, SFX, AL)          \
-    T0G_GEMM(PFX##_nt_##OUTN##SFX, BM, BN, WM, WN, true, true, OBF, AL)    \
-    T0G_GEMM(PFX##_nn_##OUTN##SFX, BM, BN, WM, WN, true, false, OBF, AL)   \
-    T0G_GEMM(PFX##_tn_##OUTN##SFX, BM, BN, WM, WN, false, false, OBF, AL)  \
-    T0G_GEMM(PFX##_tt_##OUTN##SFX, BM, BN, WM, WN, false, true, OBF, AL)
+#define T0G_GEMM_LAYOUTS(PFX, BM, BN, WM, WN, OUTN, OBF)              \
+    T0G_GEMM(PFX##_nt_##OUTN, BM, BN, WM, WN, true, true, OBF)        \
+    T0G_GEMM(PFX##_nn_##OUTN, BM, BN, WM, WN, true, false, OBF)       \
+    T0G_GEMM(PFX##_tn_##OUTN, BM, BN, WM, WN, false, false, OBF)      \
+    T0G_GEMM(PFX##_tt_##OUTN, BM, BN, WM, WN, false, true, OBF)
 
-#define T0G_GEMM_TILE(PFX, BM, BN, WM, WN)                       \
-    T0G_GEMM_LAYOUTS(PFX, BM, BN, WM, WN, f32, false, , true)    \
-    T0G_GEMM_LAYOUTS(PFX, BM, BN, WM, WN, bf16, true, , true)
+#define T0G_GEMM_TILE(PFX, BM, BN, WM, WN)             \
+    T0G_GEMM_LAYOUTS(PFX, BM, BN, WM, WN, f32, false)  \
+    T0G_GEMM_LAYOUTS(PFX, BM, BN, WM, WN, bf16, true)
 
-#define T0G_GEMM_TILE_U(PFX, BM, BN, WM, WN)                     \
-    T0G_GEMM_LAYOUTS(PFX, BM, BN, WM, WN, f32, false, _u, false) \
-    T0G_GEMM_LAYOUTS(PFX, BM, BN, WM, WN, bf16, true, _u, false)
+// Operands staged through registers (512 threads: four MFMA waves and four
+// staging waves).  D: stages in flight in VGPRs; 64x64 tiles with bf16 operands
+// and one f32 operand keep two workgroups on a CU (128 VGPRs).
+#define T0G_GEMM_STAGED(NAME, BM, BN, AK, BKM, OBF, D, WPE, AF, BF)                                           \
+    extern "C" __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))         \
+        NAME(T0gGemmArgs p) {                                                                                \
+        t0g::gemm_tile_staged<BM, BN, AK, BKM, OBF, D, AF, BF>(p);                                           \
+    }
+#define T0G_GEMM_LAYOUTS_U(PFX, BM, BN, OUTN, OBF, D, WPE)                                      \
+    T0G_GEMM_STAGED(PFX##_nt_##OUTN##_u, BM, BN, true, true, OBF, D, WPE, false, false)         \
+    T0G_GEMM_STAGED(PFX##_nn_##OUTN##_u, BM, BN, true, false, OBF, D, WPE, false, false)        \
+    T0G_GEMM_STAGED(PFX##_tn_##OUTN##_u, BM, BN, false, false, OBF, D, WPE, false, false)       \
+    T0G_GEMM_STAGED(PFX##_tt_##OUTN##_u, BM, BN, false, true, OBF, D, WPE, false, false)
+#define T0G_GEMM_TILE_U(PFX, BM, BN, D, WPE)                 \
+    T0G_GEMM_LAYOUTS_U(PFX, BM, BN, f32, false, D, WPE)      \
+    T0G_GEMM_LAYOUTS_U(PFX, BM, BN, bf16, true, D, WPE)
+// f32 operands (the Ignis caller path), rounded to bf16 on their way to LDS:
+// suffix _ff (both) or _fb (A; B already bf16), f32 out, the layouts of the
+// forward (NN), the data gradient and bf16 weights (NT) and the weight gradient (TN).
+#define T0G_GEMM_TILE_F(PFX, BM, BN, DFF, WFF, DFB, WFB)                                     \
+    T0G_GEMM_STAGED(PFX##_nn_f32_ff, BM, BN, true, false, false, DFF, WFF, true, true)       \
+    T0G_GEMM_STAGED(PFX##_nn_f32_fb, BM, BN, true, false, false, DFB, WFB, true, false)      \
+    T0G_GEMM_STAGED(PFX##_nt_f32_ff, BM, BN, true, true, false, DFF, WFF, true, true)        \
+    T0G_GEMM_STAGED(PFX##_nt_f32_fb, BM, BN, true, true, false, DFB, WFB, true, false)       \
+    T0G_GEMM_STAGED(PFX##_tn_f32_ff, BM, BN, false, false, false, DFF, WFF, true, true)
 
 // Deep-ring variants (suffix _d) of the 64x64 and 128x128 tiles for grids of
 // at most one workgroup per CU (split-K and thin shapes): 128 KB of LDS per
@@ -1596,8 +1638,11 @@ T0G_GEMM_LAYOUTS_R(t0g_gemm_128x128_k64, 128, 128, 2, 2, bf16, true)
 T0G_GEMM_LAYOUTS_256_R(f32, false)
 T0G_GEMM_LAYOUTS_256_R(bf16, true)
 T0G_GEMM_TILE(t0g_gemm_64x64_k64, 64, 64, 2, 2)
-T0G_GEMM_TILE_U(t0g_gemm_128x128_k64, 128, 128, 2, 2)
-T0G_GEMM_TILE_U(t0g_gemm_64x64_k64, 64, 64, 2, 2)
+T0G_GEMM_TILE_U(t0g_gemm_128x128_k64, 128, 128, 4, 2)
+T0G_GEMM_TILE_U(t0g_gemm_64x64_k64, 64, 64, 4, 4)
+
+T0G_GEMM_TILE_F(t0g_gemm_64x64_k64, 64, 64, 2, 4, 2, 4)
+
 T0G_GEMM_TILE_D(t0g_gemm_64x64_k64, 64, 64, 2, 2)
 T0G_GEMM_TILE_D(t0g_gemm_128x128_k64, 128, 128, 2, 2)
 

@@ -127,6 +127,11 @@ typedef struct T0gConvertArgs {
     uint32_t flags;          /* T0G_CONVERT_VEC                                   */
 } T0gConvertArgs;
 
+/* Two conversions in one launch: workgroups [0, a.grid_blocks) and the next b.grid_blocks. */
+typedef struct T0gConvertPairArgs {
+    T0gConvertArgs a, b;
+} T0gConvertPairArgs;
+
 #define T0G_FLAG_XCD_REMAP 1u   /* remap workgroup ids so each XCD owns a contiguous tile (128x128, 64x64: (split, tile)) range */
 #define T0G_FLAG_C_VEC 2u       /* C base, row pitch and split-plane stride are 16-byte aligned */
 #define T0G_FLAG_BIAS 4u        /* the chain reads bias[col]                                     */

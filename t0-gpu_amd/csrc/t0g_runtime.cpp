@@ -7,6 +7,7 @@
 // hipModuleLoadData / hipModuleLaunchKernel on a code object built ahead of
 // time by hipcc for gfx950.
 #include <hip/hip_runtime_api.h>
+#include <math.h>
 #include <stdio.h>
 #include <string.h>
 #include <time.h>
@@ -408,6 +409,7 @@ static int make_plan(const TileDef *tile, uint32_t transpose, bool out_bf16, Ope
     // the stream-K ones with a K-contiguous A (NN, NT), which keep the 8-wave
     // ping-pong schedule.
     p->wg = (tile->bm == 256 && !(stream_k && a_k_major(transpose))) ? 256u : tile->wg;
+    if (!aligned) p->wg = 512;   // staged operands: four MFMA waves and four staging waves
     // The 64x64 deep ring splits K across its four waves (_ds, _dsr) for K
     // ranges of kKsplitMinStages 64-K stages or more: the loop then reads each
     // fragment once per stage instead of twice, and the closing sum of the four
@@ -1706,11 +1708,7 @@ extern "C" {
 
 // ---- Ignis bf16_matmul caller path ------------------------------------------
 
-static int convert_locked(t0g_device *dev, uint64_t src, uint64_t dst, uint64_t n) {
-    if (n == 0) return T0G_OK;
-    hipFunction_t f = nullptr;
-    int rc = get_function(dev, "t0g_f32_to_bf16_rne", &f);
-    if (rc) return rc;
+static T0gConvertArgs convert_args(uint64_t src, uint64_t dst, uint64_t n) {
     T0gConvertArgs a;
     memset(&a, 0, sizeof a);
     a.src = src;
@@ -1724,7 +1722,94 @@ static int convert_locked(t0g_device *dev, uint64_t src, uint64_t dst, uint64_t 
     const uint64_t cap = vec ? (1u << 20) : 8192;
     if (blocks > cap) blocks = cap;
     a.grid_blocks = (uint32_t)blocks;
-    return launch(dev, f, (uint32_t)blocks, 1, 1, 256, &a, sizeof a);
+    return a;
+}
+
+static int convert_locked(t0g_device *dev, uint64_t src, uint64_t dst, uint64_t n) {
+    if (n == 0) return T0G_OK;
+    hipFunction_t f = nullptr;
+    int rc = get_function(dev, "t0g_f32_to_bf16_rne", &f);
+    if (rc) return rc;
+    T0gConvertArgs a = convert_args(src, dst, n);
+    return launch(dev, f, a.grid_blocks, 1, 1, 256, &a, sizeof a);
+}
+
+// Two operands in one launch: a launch of its own costs the smaller one 3 to 4 us,
+// its conversion beside the larger one's next to nothing.
+static int convert_pair_locked(t0g_device *dev, uint64_t src0, uint64_t dst0, uint64_t n0, uint64_t src1,
+                               uint64_t dst1, uint64_t n1) {
+    if (n0 == 0) return convert_locked(dev, src1, dst1, n1);
+    if (n1 == 0) return convert_locked(dev, src0, dst0, n0);
+    hipFunction_t f = nullptr;
+    int rc = get_function(dev, "t0g_f32_to_bf16_rne_pair", &f);
+    if (rc) return rc;
+    T0gConvertPairArgs a = {convert_args(src0, dst0, n0), convert_args(src1, dst1, n1)};
+    return launch(dev, f, a.a.grid_blocks + a.b.grid_blocks, 1, 1, 256, &a, sizeof a);
+}
+
+// One GEMM with f32 output whose A (and, with b_f32, B) is f32, rounded to bf16
+// inside the kernel (64x64 tile, gemm_staged.h).
+static int staged_f32_locked(t0g_device *dev, uint64_t a, uint64_t b, bool b_f32, uint64_t c, uint32_t m, uint32_t n,
+                             uint32_t k, uint32_t transpose, uint32_t split) {
+    GemmPlan p;
+    int rc = make_plan(&kTiles[2], transpose, false, OperandPath::Staged, true, m, n, k, split, &p);
+    if (rc) return rc;
+    p.symbol.replace(p.symbol.size() - 2, 2, b_f32 ? "_ff" : "_fb");
+    GemmOperands o;
+    memset(&o, 0, sizeof o);
+    o.a = a;
+    o.b = b;
+    o.c = c;
+    o.m = m;
+    o.n = n;
+    o.k = k;
+    o.lda = a_k_major(transpose) ? k : m;
+    o.ldb = b_k_major(transpose) ? k : n;
+    o.ldc = n;
+    uint64_t ws = 0;
+    if (p.splits > 1) {
+        if ((rc = ensure_workspace(dev, plan_workspace(p, m, n, dev->num_cus)))) return rc;
+        ws = dev->ws;
+    }
+    return run_plan(dev, p, o, ws);
+}
+
+// Whether converting inside the GEMM beats conversion launches plus the bf16
+// GEMM, and over how many K slices.  The kernel's 64-K step takes 0.5 us with two
+// f32 operands and 0.33 us with one (32 and 24 KB into each CU), so it wins where
+// the conversion's launch and pass weigh more than a slower K loop: small and
+// ordinary layers.  Converting first against inside, one box: 32x128x128 forward
+// 7.6 / 4.7 us, 1024^3 forward 14.2 / 12.1, its data gradient with a cached weight
+// 12.1 / 9.4, 512x3072x768 data gradient 18.2 / 15.0 (split 2); but 2048x2048x512
+// forward 15.6 / 20.9, 768x3072x512 weight gradient 12.5 / 15.5.
+static bool staged_f32_wins(uint32_t m, uint32_t n, uint32_t k, uint32_t transpose, bool b_f32, uint64_t conv_elems,
+                            uint32_t *split) {
+    if (m == 0 || n == 0 || k == 0) return false;
+    // 32-bit byte offsets, with room: far above any size it wins at
+    if ((uint64_t)m * k >= (1ull << 28) || (uint64_t)k * n >= (1ull << 28)) return false;
+    t0g_gemm_config cfg;
+    select_config(m, k, n, &cfg, false);
+    double conv = 3.0 + 6.0 * (double)conv_elems / 4.5e6;
+    const bool aligned = operand_path(0, 0, m, n, k, a_k_major(transpose) ? k : m, b_k_major(transpose) ? k : n,
+                                      transpose) != OperandPath::Staged;
+    // unaligned operands are staged as bf16 then, at about 0.7 of the fast kernels' rate
+    conv += model_time_us(*find_tile(cfg.tile_m, cfg.tile_n, cfg.tile_k, cfg.wg_size), m, k, n, cfg_split(&cfg)) *
+            (aligned ? 1.0 : 1.4);
+    const double tiles = (double)((m + 63) / 64) * ((n + 63) / 64), stage = b_f32 ? 0.5 : 0.33;
+    double best = 0.97 * conv;
+    bool wins = false;
+    for (uint32_t sk = 1; sk <= 8; sk *= 2) {
+        if (sk > 1 && k < sk * 4 * kTileK) break;
+        const double per_cu = tiles * sk / kNumCUs, steps = ceil((double)k / sk / kTileK);
+        double t = 3.5 + (per_cu > 1.0 ? per_cu : 1.0) * (steps * stage + 1.0);
+        if (sk > 1) t += 2.5 + (double)sk * m * n * 4.0 / 4.5e6 + 0.25 * sk;   // as model_time_us
+        if (t < best) {
+            best = t;
+            wins = true;
+            *split = sk;
+        }
+    }
+    return wins;
 }
 
 static int ensure_conv(t0g_device *dev, size_t bytes) {
@@ -1745,8 +1830,8 @@ static int ensure_conv(t0g_device *dev, size_t bytes) {
 
 static size_t round256(size_t b) { return (b + 255) & ~(size_t)255; }
 
-// Convert the f32 operands that need it into the scratch buffer, then run one
-// GEMM with f32 output.  a_elems / b_elems: elements of A and B (0: already bf16).
+// One GEMM with f32 output on f32 operands: rounded to bf16 inside the kernel, or
+// converted into the scratch buffer first (staged_f32_wins).  a_elems / b_elems: elements of A and B (0: already bf16).
 static int matmul_common(t0g_device *dev, uint64_t a_f32, size_t a_elems, uint64_t b, size_t b_elems,
                          uint64_t c, uint32_t m, uint32_t n, uint32_t k, uint32_t transpose) {
     if (!dev) return fail(T0G_ERR_INVALID_ARG, "device is NULL");
@@ -1754,11 +1839,13 @@ static int matmul_common(t0g_device *dev, uint64_t a_f32, size_t a_elems, uint64
     std::lock_guard<std::mutex> lk(dev->mu);
     int rc = check_usable(dev);
     if (rc) return rc;
+    uint32_t split = 1;
+    if (staged_f32_wins(m, n, k, transpose, b_elems != 0, a_elems + b_elems, &split))
+        return staged_f32_locked(dev, a_f32, b, b_elems != 0, c, m, n, k, transpose, split);
     const size_t a_bytes = round256(a_elems * 2), b_bytes = round256(b_elems * 2);
     if ((rc = ensure_conv(dev, a_bytes + b_bytes + 256))) return rc;
     const uint64_t a16 = dev->conv, b16 = b_elems ? dev->conv + a_bytes : b;
-    if ((rc = convert_locked(dev, a_f32, a16, a_elems))) return rc;
-    if (b_elems && (rc = convert_locked(dev, b, b16, b_elems))) return rc;
+    if ((rc = convert_pair_locked(dev, a_f32, a16, a_elems, b, b16, b_elems))) return rc;
     t0g_gemm_desc d;
     memset(&d, 0, sizeof d);
     d.a = a16;
@@ -1892,6 +1979,11 @@ static int matmul_cached(t0g_device *dev, uint64_t a_f32, size_t a_elems, uint64
     if (m == 0 || n == 0) return ok();
     uint64_t w16 = 0;
     if (w_elems && (rc = bf16_cache_get_locked(dev, w_id, w, w_elems, &w16))) return rc;
+    uint32_t split = 1;
+    if (staged_f32_wins(m, n, k, transpose, false, a_elems, &split)) {
+        if ((rc = staged_f32_locked(dev, a_f32, w16, false, c, m, n, k, transpose, split))) return rc;
+        return ok();
+    }
     if ((rc = ensure_conv(dev, round256(a_elems * 2) + 256))) return rc;
     if ((rc = convert_locked(dev, a_f32, dev->conv, a_elems))) return rc;
     t0g_gemm_desc d;

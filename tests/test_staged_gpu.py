@@ -73,3 +73,92 @@ def test_unaligned_operands(rt, layout, preset, m, n, k):
         finally:
             for x in bufs:
                 rt.free(x)
+
+
+# ---- f32 operands rounded inside the kernel (_ff, _fb) -----------------------------
+
+def _guarded_f32(rt, x):
+    host = np.concatenate([np.full(1, np.nan, np.float32), x.reshape(-1), np.full(16, np.nan, np.float32)])
+    addr = rt.upload(host)
+    return addr, addr + 4
+
+
+# (m, k, n) of the layer: the contraction is k forward, n for the data gradient, m for the
+# weight gradient; stage edges (63, 64, 65, 129 ...), rows of fewer than 4 values, ragged
+# tiles, sizes where K is split in the kernel (64 x 2048 x 64) and one that converts first
+# (300 x 1536 x 1544)
+LAYERS = [(32, 128, 128), (65, 63, 66), (64, 64, 64), (1, 65, 3), (3, 2, 130), (130, 129, 2), (127, 300, 191),
+          (64, 2048, 64), (5, 1000, 1001), (300, 1536, 1544)]
+
+
+@pytest.mark.parametrize("m,k,n", LAYERS)
+def test_f32_layers(rt, m, k, n):
+    rng = np.random.default_rng(m * 1009 + k * 31 + n)
+    x = rng.uniform(-0.5, 0.5, (m, k)).astype(np.float32)
+    w = rng.uniform(-0.5, 0.5, (k, n)).astype(np.float32)
+    dy = rng.uniform(-0.5, 0.5, (m, n)).astype(np.float32)
+    xb, wb, dyb = (o.f32_to_bf16_rne(v) for v in (x, w, dy))
+    t = np.ascontiguousarray
+    y_ref = o.gemm("NT", xb, t(wb.T), m, n, k)
+    dx_ref = o.gemm("NT", dyb, wb, m, k, n)
+    dw_ref = o.gemm("NT", t(xb.T), t(dyb.T), k, n, m)
+    bufs = []
+    try:
+        (bx, dx_), (bw, dw_), (bd, dd_) = (_guarded_f32(rt, v) for v in (x, w, dy))
+        bufs += [bx, bw, bd]
+        out = rt.alloc(max(m * n, m * k, k * n) * 4)
+        bufs.append(out)
+
+        def check(what, shape, ref, kk, call):
+            rt.memset(out, 0xFF, shape[0] * shape[1] * 4)
+            call()
+            rt.wait_idle()
+            ok, relf, maxabs, bound = o.parity(rt.read(out, shape, np.float32), ref, kk)
+            assert ok, f"{what}: relF={relf:.3e} max|d|={maxabs:.3e} bound={bound:.3e}"
+
+        check("forward", (m, n), y_ref, k, lambda: rt.matmul_f32(dx_, dw_, out, m, k, n))
+        check("data gradient", (m, k), dx_ref, n, lambda: rt.matmul_backward_data_f32(dd_, dw_, out, m, k, n))
+        check("weight gradient", (k, n), dw_ref, m, lambda: rt.matmul_backward_weight_f32(dx_, dd_, out, m, k, n))
+        check("cached forward", (m, n), y_ref, k, lambda: rt.matmul_f32_cached(dx_, dw_, 77, out, m, k, n))
+        check("cached data gradient", (m, k), dx_ref, n,
+              lambda: rt.matmul_backward_data_f32_cached(dd_, dw_, 77, out, m, k, n))
+        wt = rt.upload(t(wb.T))
+        bufs.append(wt)
+        check("bf16 weight", (m, n), y_ref, k, lambda: rt.matmul_wt_bf16_f32(dx_, wt, out, m, k, n))
+    finally:
+        rt.clear_bf16_cache()
+        for b in bufs:
+            rt.free(b)
+
+
+def test_f32_rounding_inside_the_kernel(rt):
+    """The operand conversion's integer rounding: ties to even, overflow to infinity, denormals, and a
+    NaN whose mantissa carries past the exponent becoming -0 (no special case), as t0g_f32_to_bf16."""
+    m, k, n = 64, 64, 64
+    bits = np.array([0x3F808000, 0x3F818000, 0x3F807FFF, 0x7F7FFFFF, 0xFF7FFFFF, 0x00000001, 0x00008000, 0x00018000,
+                     0x807FFFFF, 0x7FFF8001, 0xFFFFFFFF, 0x7F800000, 0x7FC00000, 0x80000000], dtype=np.uint32)
+    x = np.zeros((m, k), dtype=np.float32)
+    for i, b in enumerate(bits):   # one value per row, so a NaN or an infinity stays in its row
+        x[i, i] = np.array([b], np.uint32).view(np.float32)[0]
+    w = np.eye(k, n, dtype=np.float32)
+    dx_, dw_ = rt.upload(x), rt.upload(w)
+    out = rt.alloc(m * n * 4)
+    d16 = rt.alloc(m * k * 2)
+    try:
+        rt.matmul_f32(dx_, dw_, out, m, k, n)
+        rt.f32_to_bf16(dx_, d16, m * k)
+        rt.wait_idle()
+        y = rt.read(out, (m, n), np.float32)
+        x16 = o.bf16_to_f32(rt.read(d16, (m, k), np.uint16))
+        for i in range(len(bits)):
+            v = x16[i, i]
+            if np.isfinite(v):
+                # bf16 denormals as MFMA operands: kept or flushed, alike for every kernel
+                assert y[i, i] == v or (abs(v) < 2.0 ** -126 and y[i, i] == 0.0), f"{bits[i]:08x}: {y[i, i]} for {v}"
+            elif np.isinf(v):
+                assert y[i, i] == v and np.all(np.isnan(np.delete(y[i], i))), f"{bits[i]:08x}"
+            else:
+                assert np.all(np.isnan(y[i])), f"{bits[i]:08x}"
+    finally:
+        for b in (dx_, dw_, out, d16):
+            rt.free(b)
