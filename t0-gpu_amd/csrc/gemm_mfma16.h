@@ -313,6 +313,44 @@ __device__ __forceinline__ void mfma16_rows(f32x4_t (&acc)[SM][SN], const bf16x8
     }
 }
 
+// L2 prefetch of stages to come (T0G_FLAG_PREFETCH; a K loop of its own, so that the
+// plain loop stays as it is).  A DMA request has half a stage to
+// a stage (0.7 to 1.4 us) to land, which an L2 or Infinity Cache hit makes and HBM
+// often does not: every wave of the tile then waits at the same barrier.  So each
+// wave also touches a few 128-byte lines of the stage kPrefetchAhead + 2 stages on,
+// one load with a line per lane, in the half step that sends no DMA.  The
+// mid-stage wait leaves this stage's touch in flight (vmcnt(1)) and so waits for the
+// last stage's.  The workgroups that run on an XCD together share panels (8 x 4 or
+// 4 x 8 tiles), so each takes its share of a panel's lines: waves 0 and 1 of A's, 2
+// and 3 of B's.  Lines that no co-resident workgroup takes (ragged tile grids) are
+// only not prefetched.  Sent with the A half's DMA and waited for with it, the
+// touches cost 45 ns a stage instead of 30 where the operands are cached, and gained
+// 2 to 5 % less where they are not; two more stages ahead gained nothing.
+struct Prefetch16 {
+    uint64_t base;    // the wave's operand
+    uint32_t bytes;   // its extent
+    uint32_t kstep;   // bytes per k
+    uint32_t off;     // byte offset of the lane's line at k = 0, kOob for none
+};
+constexpr uint32_t kPrefetchAhead = 2;
+
+// Byte offset of the lane's line: lines [256 sub / share, 256 (sub + 1) / share) of a
+// stage's 256, half of them to each of two waves.
+template <bool K_MAJOR>
+__device__ __forceinline__ uint32_t prefetch_line(uint32_t row0, uint32_t ld, uint32_t share, uint32_t sub, uint32_t half,
+                                                  uint32_t lane) {
+    const uint32_t per_wave = 128u / share;
+    const uint32_t line = (sub * 2 + half) * per_wave + lane;
+    const uint32_t off = K_MAJOR ? (row0 + line) * ld * 2u : ((line >> 2) * ld + row0 + (line & 3u) * 64u) * 2u;
+    return lane < per_wave ? off : kOob;
+}
+
+// The descriptor whose words rsrc_words32 formed.
+__device__ __forceinline__ rsrc_t rsrc_of(u32x4_t w) {
+    return __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void*>(((uint64_t)w[1] << 32) | w[0]), (short)0, (int)w[2],
+                                             kRsrcWord3);
+}
+
 // K loop: two 64 KB stages of 64 K values (two 32-wide steps each).  Halfway
 // through step 1 of stage s one vmcnt(0)/lgkmcnt(0) wait and a barrier make
 // stage s + 1 visible and free the buffer of stage s; the step's second half
@@ -321,11 +359,13 @@ __device__ __forceinline__ void mfma16_rows(f32x4_t (&acc)[SM][SN], const bf16x8
 // s + 1.  Each DMA so has half a stage or more to land before it is waited on.
 // Stages past the end get an empty descriptor: their DMA writes zeros to LDS
 // and reads no memory.
-template <bool CHECK, uint32_t A_BYTES, uint32_t STAGE, int kVmemPerStage, int SM, int SN, class OpA, class OpB>
+template <bool CHECK, uint32_t A_BYTES, uint32_t STAGE, int kVmemPerStage, bool PF = false, int SM, int SN, class OpA,
+          class OpB>
 __device__ __forceinline__ void k_pipeline16(f32x4_t (&acc)[SM][SN], const OpA& la, const OpB& lb,
                                              const T0gGemmArgs& p, typename OpA::bytes_t a_bytes,
                                              typename OpB::bytes_t b_bytes, uint32_t kbeg,
-                                             uint32_t kend, int nst, uint32_t lds0) {
+                                             uint32_t kend, int nst, uint32_t lds0,
+                                             Prefetch16 pf = Prefetch16{0, 0, 0, kOob}) {
     constexpr int kHalf = OpA::kInstr;   // the A half of a stage's DMA, then the B half
     static_assert(OpA::kInstr == OpB::kInstr, "equal A and B halves");
     bf16x8_t fa0[SM], fb0[SN], fa1[SM], fb1[SN];
@@ -344,6 +384,7 @@ __device__ __forceinline__ void k_pipeline16(f32x4_t (&acc)[SM][SN], const OpA& 
 
     constexpr int kHalfRows = SM / 2;
     uint32_t cur = 0;
+    uint32_t touched = 0;
     for (int s = 0; s < nst; ++s) {
         const uint32_t nxt = cur ^ STAGE;
         const uint32_t k1 = kbeg + (uint32_t)(s + 1) * 64, k2 = k1 + 64;
@@ -351,14 +392,21 @@ __device__ __forceinline__ void k_pipeline16(f32x4_t (&acc)[SM][SN], const OpA& 
         const u32x4_t ra2 = la.rsrc(p.a, k2 < kend ? a_bytes : typename OpA::bytes_t{0}, p.lda, k2);
         mfma16_rows<0, kHalf, kHalf, CHECK, 0, SM, 0>(acc, fa0, fb0, fa1, fb1, la, lb, lds0 + cur, lds0 + nxt,
                                                      lds0 + nxt, ra2, rb1, k1, kend);
+        if constexpr (PF) {
+            const uint32_t kp = k2 + 64u * kPrefetchAhead;
+            const rsrc_t q = rsrc_of(rsrc_words32(pf.base, kp < kend ? pf.bytes : 0u, kp * pf.kstep));
+            touched = __builtin_amdgcn_raw_buffer_load_b32(q, pf.off, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+        }
         mfma16_rows<1, 0, 0, CHECK, 0, kHalfRows, kHalfRows>(acc, fa1, fb1, fa0, fb0, la, lb, lds0 + cur, lds0 + nxt,
                                                             lds0 + nxt, ra2, rb1, k1, kend);
-        __builtin_amdgcn_s_waitcnt(0x0070);   // vmcnt(0) lgkmcnt(0)
+        __builtin_amdgcn_s_waitcnt(PF ? 0x0071 : 0x0070);   // vmcnt(0), PF: all but this stage's touch; lgkmcnt(0)
         barrier_no_fence();
         mfma16_rows<1, 0, kHalf, CHECK, kHalfRows, SM, kHalfRows>(acc, fa1, fb1, fa0, fb0, la, lb, lds0 + cur,
                                                                  lds0 + nxt, lds0 + cur, ra2, rb1, k2, kend);
         cur = nxt;
     }
+    if constexpr (PF) asm volatile("" : : "v"(touched));
 }
 
 // Epilogue: each wave stages 32 rows x WTN columns of fp32 at a time through
@@ -742,9 +790,26 @@ __device__ __forceinline__ void gemm_tile_fast16(const T0gGemmArgs& p, const T0g
     if (nst > 0) {
         mfma16_drain();
         const uint32_t lds0 = __builtin_amdgcn_readfirstlane(lds_addr(smem));
-        if ((kend - kbeg) % 64 == 0)
+        const bool whole = (kend - kbeg) % 64 == 0;
+        bool plain = whole;
+        if constexpr (!WIDE && !RED) {
+            if (whole && (p.flags & T0G_FLAG_PREFETCH)) {
+                plain = false;
+                const uint32_t rows = p.tiles_m >= 8 ? 8u : p.tiles_m >= 4 ? 4u : 2u, cols = rows == 8 ? 4u : 8u;
+                const uint32_t w = __builtin_amdgcn_readfirstlane(wave);
+                Prefetch16 pf;
+                pf.off = w < 2 ? prefetch_line<A_K>(m0, p.lda, cols, (n0 / BN) % cols, w & 1u, lane)
+                               : prefetch_line<B_K>(n0, p.ldb, rows, (m0 / BM) % rows, w & 1u, lane);
+                pf.base = w < 2 ? p.a : p.b;
+                pf.bytes = w < 2 ? a_bytes : b_bytes;
+                pf.kstep = 2u * (w < 2 ? (A_K ? 1u : p.lda) : (B_K ? 1u : p.ldb));
+                k_pipeline16<false, A_BYTES, STAGE, kVmemPerStage, true>(acc, la, lb, p, a_bytes, b_bytes, kbeg, kend,
+                                                                         nst, lds0, pf);
+            }
+        }
+        if (plain)
             k_pipeline16<false, A_BYTES, STAGE, kVmemPerStage>(acc, la, lb, p, a_bytes, b_bytes, kbeg, kend, nst, lds0);
-        else
+        else if (!whole)
             k_pipeline16<true, A_BYTES, STAGE, kVmemPerStage>(acc, la, lb, p, a_bytes, b_bytes, kbeg, kend, nst, lds0);
     }
 

@@ -505,6 +505,15 @@ static void fill_gemm_args(const GemmPlan &p, const GemmOperands &o, uint64_t ws
     args.tiles_n = p.tiles_n;
     args.group_m = 8;
     args.flags = T0G_FLAG_XCD_REMAP | (allow_timeline && g_timeline.load() ? T0G_FLAG_TIMELINE : 0u);
+    // Operands of 96 MB or more come from HBM as a rule (with the output and whatever
+    // ran before, they do not stay in the 256 MiB Infinity Cache): the 256x256
+    // kernels then prefetch into the L2.  Three sets of operands in turn, without
+    // and with it: 1024 x 11008 x 4096 NN (99 MB) 88.0 / 81.5 us, NT 93.7 / 80.8, 2048 x
+    // 11008 x 4096 NT 186.9 / 168.1, 8192^3 NN 776.8 / 754.6, NT 792.6 / 749.6, 5120^3
+    // 221.0 / 216.8; below, what a prefetch costs shows: 4096^3 (67 MB) NN 95.7 / 98.0,
+    // 4096 x 5120 x 4096 (75 MB) 160.8 / 164.7, 11008 x 4096 x 1024 TN (31 MB) 83.4 / 86.0.
+    // One shape above it lost, 6144^3 NN 381.2 / 387.0 (NT 380.3 / 370.7).
+    if (p.tile->bm == 256 && 2.0 * o.k * ((double)o.m + o.n) >= 96e6) args.flags |= T0G_FLAG_PREFETCH;
     const bool reduce = p.splits > 1 && o.c_split_stride == 0 && !p.fused;
     if (reduce) {
         args.c = ws;
