@@ -918,6 +918,40 @@ __device__ __forceinline__ void k_pipeline(f32x16_t (&acc)[SM][SN], const OpA& l
 #undef T0G_KD
 }
 
+// The DMA of a k_pipeline or k_pipeline_deep loop with OWN = false, by four waves of
+// their own (the deep rings).  What bounds the 128x128 loop is how long a stage's DMA takes to land with two
+// stages of lookahead (per 64-K stage 0.446 us; without the DMA 0.33, without the MFMAs
+// 0.33): sent by the MFMA waves, a stage's eight requests per wave go out one behind
+// each of its MFMAs and so over the whole stage; these waves send all of them as soon as the
+// barrier frees the buffer.  Before and after, three sets of operands in turn:
+// 2048^3 NT 19.9 / 19.5 us, 1024x4096x4096 NN 34.7 / 33.4, 2048x2048x8192 NN 64.7 /
+// 62.1, 1024x4096x8192 NT 64.0 / 60.1, 512x3072x768 TN 8.75 / 8.61; 2048x2048x512 TN
+// 8.85 / 8.84.  On 64x64 tiles, where a wave has one MFMA per K step, the requests and
+// their descriptors were most of what a wave issued: 1024^3 NT 7.19 / 6.40, 256x256x1024
+// 6.53 / 5.59.  128x128: a fifth stage (all 160 KB) gained nothing more at K = 8192 and took
+// 2048^3 to 20.4 us; touching lines ahead as the 256x256 kernels do took it to 20.2.
+template <bool CHECK, uint32_t BK, int NS, uint32_t A_BYTES, uint32_t STAGE, int kVmemPerStage, class OpA, class OpB>
+__device__ __forceinline__ void dma_feed(const OpA& la, const OpB& lb, const T0gGemmArgs& p, uint32_t a_bytes,
+                                         uint32_t b_bytes, uint32_t kbeg, uint32_t kend, int nst, uint32_t lds0) {
+    static_assert(NS >= 4, "ring of at least 4 stages");
+#pragma unroll
+    for (int s = 0; s < NS - 1; ++s) {
+        la.template issue<CHECK>(lds0 + s * STAGE, p.a, a_bytes, p.lda, kbeg + s * BK, kend);
+        lb.template issue<CHECK>(lds0 + s * STAGE + A_BYTES, p.b, b_bytes, p.ldb, kbeg + s * BK, kend);
+    }
+    T0G_WAIT_VMCNT(kVmemPerStage * (NS - 3));   // stages 0 and 1 have landed
+    barrier_no_fence();
+    uint32_t fill = (NS - 1) * STAGE;           // buffer receiving stage s + NS - 1
+    for (int s = 0; s < nst; ++s) {
+        const uint32_t kf = kbeg + (uint32_t)(s + NS - 1) * BK;
+        la.template issue<CHECK>(lds0 + fill, p.a, a_bytes, p.lda, kf, kend);
+        lb.template issue<CHECK>(lds0 + fill + A_BYTES, p.b, b_bytes, p.ldb, kf, kend);
+        T0G_WAIT_VMCNT(kVmemPerStage * (NS - 3));   // stage s + 2 has landed
+        barrier_no_fence();
+        fill = fill + STAGE == NS * STAGE ? 0 : fill + STAGE;
+    }
+}
+
 // Deep-ring K loop of the 64x64 tile (BK 64, one workgroup per CU, one 32x32
 // MFMA block per wave): the fragments of a whole stage are read one stage
 // ahead, right after the barrier that makes the stage visible, into one of
@@ -1162,9 +1196,10 @@ namespace t0g {
 
 // Fast path: one BM x BN output tile per workgroup, operands streamed through
 // LDS by DMA (k_pipeline), epilogue staged through LDS.  RED: split-K reduced
-// inside the kernel (ra: the launch's T0gGemmRedArgs, p = ra->g).
+// inside the kernel (ra: the launch's T0gGemmRedArgs, p = ra->g).  FEED: four more waves
+// send the DMA (dma_feed).
 template <int BM, int BN, int WAVES_M, int WAVES_N, bool A_K, bool B_K, bool OUT_BF16, uint32_t BK, int NS,
-          bool RED = false, bool KS = false>
+          bool RED = false, bool KS = false, bool FEED = false>
 __device__ __forceinline__ void gemm_tile_fast(const T0gGemmArgs& p, const T0gGemmRedArgs* ra = nullptr) {
     constexpr int NT = 64 * WAVES_M * WAVES_N;
     constexpr int WTM = BM / WAVES_M, WTN = BN / WAVES_N;
@@ -1178,7 +1213,7 @@ __device__ __forceinline__ void gemm_tile_fast(const T0gGemmArgs& p, const T0gGe
     __shared__ __attribute__((aligned(1024))) char smem[NS * STAGE];
 
     tl_mark(p, 0);
-    const uint32_t tid = threadIdx.x;
+    const uint32_t tid = FEED ? threadIdx.x % NT : threadIdx.x;
     const GridPos gp = grid_pos(p);
     const uint32_t bid = gp.tile;
     const uint32_t gm = p.group_m;
@@ -1204,6 +1239,23 @@ __device__ __forceinline__ void gemm_tile_fast(const T0gGemmArgs& p, const T0gGe
     OpB lb;
     la.init(tid, m0, p.lda, wm * WTM, l32, g);
     lb.init(tid, n0, p.ldb, wn * WTN, l32, g);
+
+    if constexpr (FEED) {
+        if (__builtin_amdgcn_readfirstlane(threadIdx.x) >= (uint32_t)NT) {
+            if (nst > 0) {
+                const uint32_t lds0 = __builtin_amdgcn_readfirstlane(lds_addr(smem));
+                if ((kend - kbeg) % BK == 0)
+                    dma_feed<false, BK, NS, A_BYTES, STAGE, kVmemPerStage>(la, lb, p, a_bytes, b_bytes, kbeg, kend,
+                                                                           nst, lds0);
+                else
+                    dma_feed<true, BK, NS, A_BYTES, STAGE, kVmemPerStage>(la, lb, p, a_bytes, b_bytes, kbeg, kend,
+                                                                          nst, lds0);
+            }
+            T0G_WAIT_VMCNT(0);    // stages past K have landed
+            barrier_no_fence();   // the epilogue may have the ring
+            return;
+        }
+    }
 
     f32x16_t acc[SM][SN];
 #pragma unroll
@@ -1240,15 +1292,15 @@ __device__ __forceinline__ void gemm_tile_fast(const T0gGemmArgs& p, const T0gGe
                                                                            kend, nst, lds0);
         } else if constexpr (BK == 64 && SM * SN == 1) {
             f32x16_t(&accd)[1][SM][SN] = *reinterpret_cast<f32x16_t(*)[1][SM][SN]>(&acc);
-            if ((kend - kbeg) % BK == 0)
-                k_pipeline_deep<false, true, NS, A_BYTES, STAGE, kVmemPerStage>(accd, la, lb, p, a_bytes, b_bytes, kbeg,
+            if (FEED || (kend - kbeg) % BK == 0)
+                k_pipeline_deep<false, !FEED, NS, A_BYTES, STAGE, kVmemPerStage>(accd, la, lb, p, a_bytes, b_bytes, kbeg,
                                                                           kend, nst, lds0);
             else
                 k_pipeline_deep<true, true, NS, A_BYTES, STAGE, kVmemPerStage>(accd, la, lb, p, a_bytes, b_bytes, kbeg,
                                                                          kend, nst, lds0);
         } else {
-            if ((kend - kbeg) % BK == 0)
-                k_pipeline<false, true, BK, NS, A_BYTES, STAGE, kVmemPerStage>(acc, la, lb, p, a_bytes, b_bytes, kbeg,
+            if (FEED || (kend - kbeg) % BK == 0)
+                k_pipeline<false, !FEED, BK, NS, A_BYTES, STAGE, kVmemPerStage>(acc, la, lb, p, a_bytes, b_bytes, kbeg,
                                                                           kend, nst, lds0);
             else
                 k_pipeline<true, true, BK, NS, A_BYTES, STAGE, kVmemPerStage>(acc, la, lb, p, a_bytes, b_bytes, kbeg,
@@ -1552,19 +1604,23 @@ extern "C" __global__ void __launch_bounds__(256) t0g_f32_to_bf16_rne_pair(T0gCo
 // flight; 128x128: 4 stages, 3 in flight.
 #define T0G_PIPE_D_64x64 64, 8
 #define T0G_PIPE_D_128x128 64, 4
-#define T0G_GEMM_D(NAME, BM, BN, WM, WN, AK, BKM, OBF)                                                           \
-    extern "C" __global__ void __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(1, 1)))       \
-        NAME(T0gGemmArgs p) {                                                                                  \
-        t0g::gemm_tile_fast<BM, BN, WM, WN, AK, BKM, OBF, T0G_PIPE_D_##BM##x##BN>(p);                           \
+// FEED 1: four more waves send the DMA (dma_feed).  bf16 output is never split, so its
+// kernels all have them; f32 has both, _df for products and _d for split planes, whose
+// short slices gained nothing (128x4096x4096 NN on 128x128, split 8: 16.95 / 16.91 us).
+#define T0G_GEMM_D(NAME, BM, BN, WM, WN, AK, BKM, OBF, FEED)                                                   \
+    extern "C" __global__ void __launch_bounds__(64 * WM * WN * (1 + FEED))                                    \
+        __attribute__((amdgpu_waves_per_eu(1 + FEED, 1 + FEED))) NAME(T0gGemmArgs p) {                         \
+        t0g::gemm_tile_fast<BM, BN, WM, WN, AK, BKM, OBF, T0G_PIPE_D_##BM##x##BN, false, false, FEED != 0>(p); \
     }
-#define T0G_GEMM_LAYOUTS_D(PFX, BM, BN, WM, WN, OUTN, OBF)                  \
-    T0G_GEMM_D(PFX##_nt_##OUTN##_d, BM, BN, WM, WN, true, true, OBF)        \
-    T0G_GEMM_D(PFX##_nn_##OUTN##_d, BM, BN, WM, WN, true, false, OBF)       \
-    T0G_GEMM_D(PFX##_tn_##OUTN##_d, BM, BN, WM, WN, false, false, OBF)      \
-    T0G_GEMM_D(PFX##_tt_##OUTN##_d, BM, BN, WM, WN, false, true, OBF)
-#define T0G_GEMM_TILE_D(PFX, BM, BN, WM, WN)                \
-    T0G_GEMM_LAYOUTS_D(PFX, BM, BN, WM, WN, f32, false)     \
-    T0G_GEMM_LAYOUTS_D(PFX, BM, BN, WM, WN, bf16, true)
+#define T0G_GEMM_LAYOUTS_D(PFX, BM, BN, WM, WN, OUTN, OBF, FEED)            \
+    T0G_GEMM_D(PFX##_nt_##OUTN, BM, BN, WM, WN, true, true, OBF, FEED)      \
+    T0G_GEMM_D(PFX##_nn_##OUTN, BM, BN, WM, WN, true, false, OBF, FEED)     \
+    T0G_GEMM_D(PFX##_tn_##OUTN, BM, BN, WM, WN, false, false, OBF, FEED)    \
+    T0G_GEMM_D(PFX##_tt_##OUTN, BM, BN, WM, WN, false, true, OBF, FEED)
+#define T0G_GEMM_TILE_D(PFX, BM, BN, WM, WN)                  \
+    T0G_GEMM_LAYOUTS_D(PFX, BM, BN, WM, WN, f32_d, false, 0)  \
+    T0G_GEMM_LAYOUTS_D(PFX, BM, BN, WM, WN, f32_df, false, 1) \
+    T0G_GEMM_LAYOUTS_D(PFX, BM, BN, WM, WN, bf16_d, true, 1)
 
 // 256x256: the 4-wave kernel (one wave of 128x128 per SIMD) for every layout.
 #define T0G_GEMM_256(NAME, AK, BKM, OBF)                                                                  \

@@ -418,7 +418,14 @@ static int make_plan(const TileDef *tile, uint32_t transpose, bool out_bf16, Ope
     // 16 stages (256x256x1024 NT) 6.76 against 6.64 us; 4 stages (256^3)
     // 4.91 against 4.30 us.
     const bool ksplit = deep && tile->bm == 64 && (kps + 63) / 64 >= kKsplitMinStages;
-    const char *deep_sfx = ksplit ? (p->fused ? "_dsr" : "_ds") : (p->fused ? "_dr" : "_d");
+    // Other products on the deep rings send the DMA from four waves of its own (the
+    // f32 kernels' _df; bf16 ones all do).  Per call, without and with: 256^3 NT 4.07 /
+    // 3.96 us, 512^3 NT 4.97 / 4.57, 1024^3 NT 7.19 / 6.40, 32x2048x1408 NT 8.17 / 6.87,
+    // 16x4096x1024 NN 7.17 / 6.16, 128^3 3.81 / 3.85; 128x128: 1024x4096x8192 NT 63.1 / 59.7,
+    // 2048^3 NN 22.8 / 22.5, 2048x2048x256 TN 7.25 / 7.24.  _ds gains nothing from it.
+    const bool feed = deep && !ksplit && !partial;
+    if (feed) p->wg = 512;
+    const char *deep_sfx = ksplit ? (p->fused ? "_dsr" : "_ds") : p->fused ? "_dr" : feed && !out_bf16 ? "_df" : "_d";
     p->symbol = std::string(tile->symbol_prefix) + "_" + layout_tag(transpose) + "_" +
                 ((out_bf16 && (!partial || p->fused)) ? "bf16" : "f32") +
                 (aligned ? (wide ? "_x" : deep ? deep_sfx : p->fused ? "_r" : "") : "_u") + (stream_k ? "_sk" : "");
