@@ -61,7 +61,8 @@ struct t0g_kernel {
     t0g::KernelKind kind;
     t0g_gemm_config cfg;          // GemmGen / TileGemm
     hipFunction_t fn = nullptr;   // Raw
-    uint32_t wg[3] = {1, 1, 1};
+    uint32_t wg[3] = {1, 1, 1};   // the unit of a dispatch's grid
+    uint32_t block_x = 1;         // Raw: threads launched along x (wg[0], or with the waves a caller left out)
     uint32_t lds = 0;
     uint32_t dyn_lds = 0;         // Raw: LDS requested at launch beyond the kernel's static LDS
     uint32_t kernarg_size = 0;    // Raw: exact argument block size, from the code object's metadata
@@ -1173,6 +1174,13 @@ int t0g_kernel_load(t0g_device *dev, const void *code_object, size_t size, const
     memset(&k->cfg, 0, sizeof k->cfg);
     k->fn = f;
     for (int i = 0; i < 3; i++) k->wg[i] = workgroup_size[i] ? workgroup_size[i] : 1;
+    // The 64x64 and 128x128 kernels built for 512 threads have four waves that only
+    // bring the operands to LDS.  256 threads, the tile's config's workgroup, still
+    // name the same workgroups: the launch adds those waves.
+    const bool mfma_waves_only = threads == 256 && k->wg[0] == 256 && meta.max_workgroup_size == 512 &&
+                                 (strncmp(symbol, "t0g_gemm_64x64_", 15) == 0 ||
+                                  strncmp(symbol, "t0g_gemm_128x128_", 17) == 0);
+    k->block_x = mfma_waves_only ? 512 : k->wg[0];
     k->lds = lds_size > meta.group_segment_size ? lds_size : meta.group_segment_size;
     k->dyn_lds = lds_size > meta.group_segment_size ? lds_size - meta.group_segment_size : 0;
     k->kernarg_size = meta.explicit_args_size;
@@ -1406,7 +1414,7 @@ static int dispatch_common(t0g_device *dev, const t0g_kernel *kernel, const uint
         size_t sz = len;
         void *extra[] = {HIP_LAUNCH_PARAM_BUFFER_POINTER, buf.data(), HIP_LAUNCH_PARAM_BUFFER_SIZE, &sz,
                          HIP_LAUNCH_PARAM_END};
-        hipError_t e = T0G_HIP(hipModuleLaunchKernel(kernel->fn, grid[0] / bx, grid[1] / by, grid[2] / bz, bx, by, bz,
+        hipError_t e = T0G_HIP(hipModuleLaunchKernel(kernel->fn, grid[0] / bx, grid[1] / by, grid[2] / bz, kernel->block_x, by, bz,
                                                      kernel->dyn_lds, dev->stream, nullptr, extra));
         if (e != hipSuccess) return poison(dev, hip_fail(e, "hipModuleLaunchKernel"));
     } else {

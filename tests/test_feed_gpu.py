@@ -61,3 +61,30 @@ def test_deep_kernels_equal_the_ordinary_one(rt, tile, layout, m, k, split):
     finally:
         for x in (da, db, dc, dh):
             rt.free(x)
+
+
+@pytest.mark.parametrize("k,out,suffix", [(320, t0g.F32, "_df"), (320, t0g.BF16, "_d"), (321, t0g.F32, "_u")])
+def test_loaded_with_the_configs_workgroup(rt, k, out, suffix):
+    """A kernel with operand waves, loaded from the code object with the 256 threads of its
+    tile's config: the same workgroups run, those waves included, and the same bits come out."""
+    m, n = 136, 200
+    rng = np.random.default_rng(k)
+    a = o.f32_to_bf16_rne(rng.uniform(-0.5, 0.5, m * k).astype(np.float32))
+    b = o.f32_to_bf16_rne(rng.uniform(-0.5, 0.5, n * k).astype(np.float32))
+    da, db = rt.upload(a), rt.upload(b)
+    dc, dr = rt.alloc(m * n * 4), rt.alloc(m * n * 4)
+    try:
+        ck = t0g.gemm_compile(t0g.gemm_desc(da, db, dc, m, n, k, out_dtype=out))
+        name, tiles = ck.name.decode(), ck.grid[0] // ck.workgroup_size
+        assert name.endswith(suffix) and ck.workgroup_size == 512
+        kern = rt.load_kernel(ck.elf(), name, (256, 1, 1), ck.lds_size)
+        dt = np.uint32 if out == t0g.F32 else np.uint16
+        for buf in (dc, dr):
+            rt.memset(buf, 0xFF, m * n * dt().itemsize)
+        rt.dispatch(kern, (tiles * 256, 1, 1), ck.args())
+        rt.gemm(da, db, dr, m, n, k, out_dtype=out)
+        rt.wait_idle()
+        assert np.array_equal(rt.read(dc, (m, n), dt), rt.read(dr, (m, n), dt))
+    finally:
+        for x in (da, db, dc, dr):
+            rt.free(x)
