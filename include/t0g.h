@@ -420,9 +420,11 @@ T0G_API int t0g_gemm_compile(const t0g_gemm_desc *desc, t0g_compiled_kernel *out
 /* ---- Ignis bf16_matmul caller path on f32 device tensors ------------------- *
  * src/ignis/ops/bf16_matmul.rs converts its f32 operands to bf16 on the CPU,
  * transposes and pads them there, runs an NT GEMM and unpads the result with a
- * second kernel.  Here the conversion runs on the GPU (t0g_f32_to_bf16, the
- * same rounding) into a library-managed scratch buffer, and the GEMM uses the
- * layout the operands already have (NN / NT / TN), unpadded: Y is written at
+ * second kernel.  Here the rounding (t0g_f32_to_bf16's) runs on the GPU: inside
+ * the GEMM for small and ordinary layers, by a conversion into a library-managed
+ * scratch buffer for the others.  The GEMM uses the layout the operands already
+ * have (NN / NT / TN), unpadded.  The output may lie over an f32 operand, whole or
+ * in part (Y over X, dX over dY); such a call always converts first.  Y is written at
  * its final [rows][cols] stride.  All pointers are device addresses of packed
  * row-major arrays; the calls are asynchronous on the device stream. */
 

@@ -1854,8 +1854,16 @@ static int ensure_conv(t0g_device *dev, size_t bytes) {
 
 static size_t round256(size_t b) { return (b + 255) & ~(size_t)255; }
 
+// Whether C shares bytes with an f32 operand of `elems` values.  The kernels that round
+// inside the GEMM read the caller's operands while other workgroups store C, so such
+// a call converts first: C may lie over its f32 operands (Y over X, dX over dY).
+static bool c_over_operand(uint64_t c, uint32_t m, uint32_t n, uint64_t operand, size_t elems) {
+    return c < operand + (uint64_t)elems * 4 && operand < c + (uint64_t)m * n * 4;
+}
+
 // One GEMM with f32 output on f32 operands: rounded to bf16 inside the kernel, or
-// converted into the scratch buffer first (staged_f32_wins).  a_elems / b_elems: elements of A and B (0: already bf16).
+// converted into the scratch buffer first (staged_f32_wins, c_over_operand).
+// a_elems / b_elems: elements of A and B (0: already bf16).
 static int matmul_common(t0g_device *dev, uint64_t a_f32, size_t a_elems, uint64_t b, size_t b_elems,
                          uint64_t c, uint32_t m, uint32_t n, uint32_t k, uint32_t transpose) {
     if (!dev) return fail(T0G_ERR_INVALID_ARG, "device is NULL");
@@ -1864,7 +1872,8 @@ static int matmul_common(t0g_device *dev, uint64_t a_f32, size_t a_elems, uint64
     int rc = check_usable(dev);
     if (rc) return rc;
     uint32_t split = 1;
-    if (staged_f32_wins(m, n, k, transpose, b_elems != 0, a_elems + b_elems, &split))
+    if (!c_over_operand(c, m, n, a_f32, a_elems) && !c_over_operand(c, m, n, b, b_elems) &&
+        staged_f32_wins(m, n, k, transpose, b_elems != 0, a_elems + b_elems, &split))
         return staged_f32_locked(dev, a_f32, b, b_elems != 0, c, m, n, k, transpose, split);
     const size_t a_bytes = round256(a_elems * 2), b_bytes = round256(b_elems * 2);
     if ((rc = ensure_conv(dev, a_bytes + b_bytes + 256))) return rc;
@@ -2004,7 +2013,7 @@ static int matmul_cached(t0g_device *dev, uint64_t a_f32, size_t a_elems, uint64
     uint64_t w16 = 0;
     if (w_elems && (rc = bf16_cache_get_locked(dev, w_id, w, w_elems, &w16))) return rc;
     uint32_t split = 1;
-    if (staged_f32_wins(m, n, k, transpose, false, a_elems, &split)) {
+    if (!c_over_operand(c, m, n, a_f32, a_elems) && staged_f32_wins(m, n, k, transpose, false, a_elems, &split)) {
         if ((rc = staged_f32_locked(dev, a_f32, w16, false, c, m, n, k, transpose, split))) return rc;
         return ok();
     }

@@ -162,3 +162,60 @@ def test_f32_rounding_inside_the_kernel(rt):
     finally:
         for b in (dx_, dw_, out, d16):
             rt.free(b)
+
+
+# (m, k, n), the call, the operand that the output lies over and by how many values it starts
+# past it: layers small enough to be rounded inside the GEMM and one that is converted first
+OVERLAPS = [(512, 512, 512, "forward", "x", 0), (1024, 1024, 1024, "forward", "x", 0),
+            (1024, 1024, 1024, "forward", "w", 0), (1024, 1024, 1024, "forward", "x", 4096),
+            (1024, 1024, 1024, "forward", "w", -4096), (1024, 1024, 1024, "cached forward", "x", 0),
+            (1024, 1024, 1024, "bf16 weight", "x", 0), (1024, 1024, 1024, "data gradient", "dy", 0),
+            (1024, 1024, 1024, "data gradient", "w", 0), (1024, 1024, 1024, "cached data gradient", "dy", 0),
+            (1024, 1024, 1024, "weight gradient", "x", 0), (1024, 1024, 1024, "weight gradient", "dy", 0),
+            (512, 768, 3072, "cached forward", "x", 0), (2001, 333, 1777, "bf16 weight", "x", 0),
+            (2001, 1777, 333, "cached data gradient", "dy", 0), (640, 512, 512, "forward", "x", 0), (65, 63, 63, "forward", "x", 0), (2048, 2048, 2048, "forward", "x", 0)]
+
+
+@pytest.mark.parametrize("m,k,n,call,over,shift", OVERLAPS)
+def test_f32_output_over_an_operand(rt, m, k, n, call, over, shift):
+    """The f32 calls take a private copy of an operand that their output lies over, so the
+    result is that of separate buffers."""
+    rng = np.random.default_rng(m + 3 * k + 5 * n + len(call))
+    host = {"x": rng.uniform(-0.5, 0.5, (m, k)).astype(np.float32),
+            "w": rng.uniform(-0.5, 0.5, (k, n)).astype(np.float32),
+            "dy": rng.uniform(-0.5, 0.5, (m, n)).astype(np.float32)}
+    t = np.ascontiguousarray
+    xb, wb, dyb = (o.f32_to_bf16_rne(host[v]) for v in ("x", "w", "dy"))
+    shape, ref, kk = {"forward": ((m, n), (xb, t(wb.T)), k), "data gradient": ((m, k), (dyb, wb), n),
+                      "weight gradient": ((k, n), (t(xb.T), t(dyb.T)), m)}[
+                          call.replace("cached ", "").replace("bf16 weight", "forward")]
+    ref = o.gemm("NT", *ref, shape[0], shape[1], kk)
+    guard = 8192
+    bufs, at = [], {}
+    try:
+        for v, a in host.items():   # room on both sides, so that a shifted output stays inside the buffer
+            room = max(a.size, shape[0] * shape[1]) + 2 * guard
+            b = rt.alloc(room * 4)
+            bufs.append(b)
+            at[v] = b + 4 * guard
+        wt = rt.upload(t(wb.T))
+        bufs.append(wt)
+        out = at[over] + 4 * shift
+        x, w, dy = at["x"], at["w"], at["dy"]
+        run = {"forward": lambda: rt.matmul_f32(x, w, out, m, k, n),
+               "cached forward": lambda: rt.matmul_f32_cached(x, w, 91, out, m, k, n),
+               "bf16 weight": lambda: rt.matmul_wt_bf16_f32(x, wt, out, m, k, n),
+               "data gradient": lambda: rt.matmul_backward_data_f32(dy, w, out, m, k, n),
+               "cached data gradient": lambda: rt.matmul_backward_data_f32_cached(dy, w, 91, out, m, k, n),
+               "weight gradient": lambda: rt.matmul_backward_weight_f32(x, dy, out, m, k, n)}[call]
+        for _ in range(5):
+            for v, a in host.items():
+                rt.write(at[v], a)
+            run()
+            rt.wait_idle()
+            ok, relf, maxabs, bound = o.parity(rt.read(out, shape, np.float32), ref, kk)
+            assert ok, f"relF={relf:.3e} max|d|={maxabs:.3e} bound={bound:.3e}"
+    finally:
+        rt.clear_bf16_cache()
+        for b in bufs:
+            rt.free(b)
