@@ -132,6 +132,10 @@ typedef struct T0gConvertPairArgs {
     T0gConvertArgs a, b;
 } T0gConvertPairArgs;
 
+/* Tiles along grid x of the kernels that stage their operands through registers; further
+ * ones go along z.  Their 512 threads would pass a grid's 2^32 threads along x from 2^23 tiles. */
+#define T0G_STAGED_TILES_X (1u << 22)
+
 #define T0G_FLAG_XCD_REMAP 1u   /* remap workgroup ids so each XCD owns a contiguous tile (128x128, 64x64: (split, tile)) range */
 #define T0G_FLAG_C_VEC 2u       /* C base, row pitch and split-plane stride are 16-byte aligned */
 #define T0G_FLAG_BIAS 4u        /* the chain reads bias[col]                                     */

@@ -437,6 +437,25 @@ static int make_plan(const TileDef *tile, uint32_t transpose, bool out_bf16, Ope
     return T0G_OK;
 }
 
+// Workgroups of a plan's launch.  The staged kernels' tiles past T0G_STAGED_TILES_X
+// go along z: 1 x 600,000,000 x 3 has 9.4 Mi tiles of 64 columns, 4.8e9 threads.
+static void plan_grid(const GemmPlan &p, uint32_t grid[3]) {
+    const uint32_t tiles = p.tiles_m * p.tiles_n;
+    const bool along_z = !p.aligned && tiles > T0G_STAGED_TILES_X;
+    grid[0] = along_z ? T0G_STAGED_TILES_X : tiles;
+    grid[1] = p.splits;
+    grid[2] = along_z ? (tiles + T0G_STAGED_TILES_X - 1) / T0G_STAGED_TILES_X : 1;
+}
+
+// A launch takes less than 2^32 threads along x; the staged kernels keep the tile
+// count of 256-thread workgroups.  Refused here, before the launch: one that fails
+// poisons the handle.
+static int check_grid(const GemmPlan &p) {
+    if ((uint64_t)p.tiles_m * p.tiles_n * (p.aligned ? p.wg : 256u) > 0xFFFFFFFFull)
+        return fail(T0G_ERR_INVALID_ARG, "%u x %u tiles: the grid in threads exceeds 32 bits", p.tiles_m, p.tiles_n);
+    return T0G_OK;
+}
+
 // The staged kernels (operands the fast path cannot take) use 32-bit byte
 // offsets.
 static int check_extent(const char *what, uint64_t rows, uint64_t ld) {
@@ -555,11 +574,13 @@ static void fill_gemm_args(const GemmPlan &p, const GemmOperands &o, uint64_t ws
 // the partial planes go to `ws` and the reduce kernel produces C.
 static int run_plan(t0g_device *dev, const GemmPlan &p, const GemmOperands &o, uint64_t ws,
                     bool allow_timeline = true) {
+    int rc = check_grid(p);
+    if (rc) return rc;
     T0gGemmArgs args;
     bool reduce = false;
     fill_gemm_args(p, o, ws, &args, &reduce, allow_timeline);
     hipFunction_t f = nullptr;
-    int rc = get_function(dev, p.symbol, &f, (args.flags & T0G_FLAG_TIMELINE) != 0);
+    rc = get_function(dev, p.symbol, &f, (args.flags & T0G_FLAG_TIMELINE) != 0);
     if (rc) return rc;
     if (p.fused) {
         T0gGemmRedArgs ra;
@@ -588,7 +609,9 @@ static int run_plan(t0g_device *dev, const GemmPlan &p, const GemmOperands &o, u
         dev->sk_stream = dev->stream;
         return launch(dev, f, sa.grid, 1, 1, p.wg, &sa, sizeof sa);
     }
-    rc = launch(dev, f, p.tiles_m * p.tiles_n, p.splits, 1, p.wg, &args, sizeof args);
+    uint32_t grid[3];
+    plan_grid(p, grid);
+    rc = launch(dev, f, grid[0], grid[1], grid[2], p.wg, &args, sizeof args);
     if (rc || !reduce) return rc;
 
     hipFunction_t fr = nullptr;
@@ -1495,8 +1518,7 @@ int t0g_gemm_compile(const t0g_gemm_desc *d, t0g_compiled_kernel *out) {
             return fail(T0G_ERR_UNSUPPORTED_CONFIG, "an epilogue cannot be applied to split-K partial planes");
         o.c_split_stride = (uint64_t)o.m * o.ldc * 4;
     }
-    if ((uint64_t)p.tiles_m * p.tiles_n * p.wg > 0xFFFFFFFFull)
-        return fail(T0G_ERR_INVALID_ARG, "%u x %u tiles: the grid in threads exceeds 32 bits", p.tiles_m, p.tiles_n);
+    if ((rc = check_grid(p))) return rc;
     T0gGemmArgs args;
     bool reduce = false;
     fill_gemm_args(p, o, 0, &args, &reduce);
@@ -1512,9 +1534,8 @@ int t0g_gemm_compile(const t0g_gemm_desc *d, t0g_compiled_kernel *out) {
     out->workgroup_size = p.wg;
     out->lds_size = meta.group_segment_size;
     out->kernarg_size = (uint32_t)sizeof args;
-    out->grid[0] = p.tiles_m * p.tiles_n * p.wg;
-    out->grid[1] = p.splits;
-    out->grid[2] = 1;
+    plan_grid(p, out->grid);
+    out->grid[0] *= p.wg;
     out->splits = p.splits;
     memcpy(out->kernargs, &args, sizeof args);
     return ok();
@@ -1638,7 +1659,8 @@ int t0g_gemm_group(t0g_device *dev, const t0g_gemm_desc *descs, uint32_t n) {
         t0g_gemm_config cfg;
         GemmPlan p;
         GemmOperands o;
-        if ((rc = resolve_desc(&descs[i], &cfg, &p, &o))) return fail(rc, "descs[%u]: %s", i, g_last_error.c_str());
+        if ((rc = resolve_desc(&descs[i], &cfg, &p, &o)) || (rc = check_grid(p)))
+            return fail(rc, "descs[%u]: %s", i, g_last_error.c_str());
     }
     if ((e = T0G_HIP(hipEventRecord(dev->fork_ev, dev->stream))) != hipSuccess)
         return poison(dev, hip_fail(e, "hipEventRecord(fork)"));

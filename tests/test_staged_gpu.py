@@ -75,6 +75,37 @@ def test_unaligned_operands(rt, layout, preset, m, n, k):
                 rt.free(x)
 
 
+def test_more_tiles_than_a_grid_row(rt):
+    """More 64-column tiles than 2^32 threads hold in 512-thread workgroups: the rest of them
+    along grid z.  One row times a column vector of repeating values, so C repeats as well."""
+    period, n = 65521, (1 << 29) + 64 * 5 + 3
+    rng = np.random.default_rng(7)
+    col = o.f32_to_bf16_rne(rng.uniform(-0.5, 0.5, period).astype(np.float32))
+    a = o.f32_to_bf16_rne(np.array([0.6875], np.float32))
+    want = o.f32_to_bf16_rne(o.bf16_to_f32(col) * np.float32(0.6875))
+    cfg = t0g.GemmConfig.preset("gfx950_64x64_k64")
+    da, db, dc = rt.upload(a), rt.upload(np.resize(col, n)), rt.alloc(n * 2)
+    try:
+        kw = dict(out_dtype=t0g.BF16, config=cfg)
+        assert t0g.gemm_compile(t0g.gemm_desc(da, db, dc, 1, n, 1, **kw)).grid[2] == 3
+        rt.memset(dc, 0xFF, n * 2)
+        rt.gemm(da, db, dc, 1, n, 1, **kw)
+        rt.wait_idle()
+        c = rt.read(dc, (n,), np.uint16)
+        whole = n - n % period
+        assert np.all(c[:whole].reshape(-1, period) == want) and np.array_equal(c[whole:], want[:n % period])
+        # one tile count further than a grid takes: refused, and the handle goes on working
+        with pytest.raises(t0g.T0gError) as e:
+            rt.gemm(da, db, dc, 1, 1 << 30, 1, **kw)
+        assert e.value.code == t0g.ERR_INVALID_ARG and not rt.is_poisoned()
+        rt.gemm(da, db, dc, 1, 5, 1, **kw)
+        rt.wait_idle()
+        assert np.array_equal(rt.read(dc, (5,), np.uint16), want[:5])
+    finally:
+        for x in (da, db, dc):
+            rt.free(x)
+
+
 # ---- f32 operands rounded inside the kernel (_ff, _fb) -----------------------------
 
 def _guarded_f32(rt, x):
