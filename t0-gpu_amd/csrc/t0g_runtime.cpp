@@ -1415,7 +1415,9 @@ static int dispatch_gemm(t0g_device *dev, const t0g_kernel *kn, const uint32_t g
     p.tiles_n = tiles_n;
     p.splits = sk;
     p.k_per_split = sk > 1 ? o.k / sk : (o.k ? o.k : kTileK);
-    if (tiles_m == 0 || tiles_n == 0) return ok();
+    // N == 0 under a grid of tiles: nothing to store, and no column for the staged
+    // kernels to clamp their loads to
+    if (tiles_m == 0 || tiles_n == 0 || o.n == 0) return ok();
     return run_plan(dev, p, o, 0);
 }
 

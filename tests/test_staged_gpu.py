@@ -106,6 +106,24 @@ def test_more_tiles_than_a_grid_row(rt):
             rt.free(x)
 
 
+@pytest.mark.parametrize("preset", ["gfx950_64x64_k64", "gfx950_128x128_k64"])
+@pytest.mark.parametrize("layout", ["NT", "NN"])
+@pytest.mark.parametrize("k", [5, 64, 333])
+def test_dispatch_of_no_columns(rt, layout, preset, k):
+    """Kernargs with N = 0 under a grid of tiles: nothing is read or stored."""
+    m = 70
+    cfg = t0g.GemmConfig.preset(preset).copy(transpose=t0g.LAYOUTS[layout])
+    kern = rt.ensure_tile_kernel(cfg)
+    da, db, dc = rt.alloc(m * k * 2), rt.alloc(256), rt.alloc(4096)
+    try:
+        rt.memset(dc, 0xA5, 4096)
+        rt.dispatch(kern, t0g.tile_compute_grid(cfg, m, 2 * cfg.tile_n), t0g.build_kernargs_m(da, db, dc, k, 0, m, cfg))
+        assert np.all(rt.read(dc, (4096,), np.uint8) == 0xA5)
+    finally:
+        for x in (da, db, dc):
+            rt.free(x)
+
+
 # ---- f32 operands rounded inside the kernel (_ff, _fb) -----------------------------
 
 def _guarded_f32(rt, x):
