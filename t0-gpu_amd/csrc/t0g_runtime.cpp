@@ -1795,13 +1795,26 @@ static int convert_pair_locked(t0g_device *dev, uint64_t src0, uint64_t dst0, ui
     return launch(dev, f, a.a.grid_blocks + a.b.grid_blocks, 1, 1, 256, &a, sizeof a);
 }
 
+// Whether the device stream is being captured into a graph: a call must not allocate then.
+static bool capturing(t0g_device *dev) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    return T0G_HIP(hipStreamIsCapturing(dev->stream, &st)) != hipSuccess || st != hipStreamCaptureStatusNone;
+}
+
 // One GEMM with f32 output whose A (and, with b_f32, B) is f32, rounded to bf16
-// inside the kernel (64x64 tile, gemm_staged.h).
+// inside the kernel (64x64 tile, gemm_staged.h).  Without the memory for its planes
+// (a workspace that would grow under capture, or cannot grow) it runs unsplit.
 static int staged_f32_locked(t0g_device *dev, uint64_t a, uint64_t b, bool b_f32, uint64_t c, uint32_t m, uint32_t n,
                              uint32_t k, uint32_t transpose, uint32_t split) {
     GemmPlan p;
     int rc = make_plan(&kTiles[2], transpose, false, OperandPath::Staged, true, m, n, k, split, &p);
     if (rc) return rc;
+    if (p.splits > 1) {
+        const size_t need = plan_workspace(p, m, n, dev->num_cus);
+        rc = dev->ws_bytes < need && capturing(dev) ? (int)T0G_ERR_OUT_OF_MEMORY : ensure_workspace(dev, need);
+        if (rc && rc != T0G_ERR_OUT_OF_MEMORY) return rc;
+        if (rc && (rc = make_plan(&kTiles[2], transpose, false, OperandPath::Staged, true, m, n, k, 1, &p))) return rc;
+    }
     p.symbol.replace(p.symbol.size() - 2, 2, b_f32 ? "_ff" : "_fb");
     GemmOperands o;
     memset(&o, 0, sizeof o);
@@ -1814,12 +1827,13 @@ static int staged_f32_locked(t0g_device *dev, uint64_t a, uint64_t b, bool b_f32
     o.lda = a_k_major(transpose) ? k : m;
     o.ldb = b_k_major(transpose) ? k : n;
     o.ldc = n;
-    uint64_t ws = 0;
-    if (p.splits > 1) {
-        if ((rc = ensure_workspace(dev, plan_workspace(p, m, n, dev->num_cus)))) return rc;
-        ws = dev->ws;
-    }
-    return run_plan(dev, p, o, ws);
+    return run_plan(dev, p, o, p.splits > 1 ? dev->ws : 0);
+}
+
+// What the staged f32 kernels take: 32-bit byte offsets, with room (far above any size
+// they win at).
+static bool staged_f32_fits(uint32_t m, uint32_t n, uint32_t k) {
+    return m != 0 && n != 0 && k != 0 && (uint64_t)m * k < (1ull << 28) && (uint64_t)k * n < (1ull << 28);
 }
 
 // Whether converting inside the GEMM beats conversion launches plus the bf16
@@ -1832,9 +1846,7 @@ static int staged_f32_locked(t0g_device *dev, uint64_t a, uint64_t b, bool b_f32
 // forward 15.6 / 20.9, 768x3072x512 weight gradient 12.5 / 15.5.
 static bool staged_f32_wins(uint32_t m, uint32_t n, uint32_t k, uint32_t transpose, bool b_f32, uint64_t conv_elems,
                             uint32_t *split) {
-    if (m == 0 || n == 0 || k == 0) return false;
-    // 32-bit byte offsets, with room: far above any size it wins at
-    if ((uint64_t)m * k >= (1ull << 28) || (uint64_t)k * n >= (1ull << 28)) return false;
+    if (!staged_f32_fits(m, n, k)) return false;
     t0g_gemm_config cfg;
     select_config(m, k, n, &cfg, false);
     double conv = 3.0 + 6.0 * (double)conv_elems / 4.5e6;
@@ -1885,6 +1897,16 @@ static bool c_over_operand(uint64_t c, uint32_t m, uint32_t n, uint64_t operand,
     return c < operand + (uint64_t)elems * 4 && operand < c + (uint64_t)m * n * 4;
 }
 
+// Whether a call's operands are rounded inside the GEMM, and over how many K slices:
+// where that wins, and under capture also where a conversion scratch of conv_bytes is
+// not there yet (a layer that ran before may have needed none).
+static bool staged_f32(t0g_device *dev, uint32_t m, uint32_t n, uint32_t k, uint32_t transpose, bool b_f32,
+                       uint64_t conv_elems, size_t conv_bytes, uint32_t *split) {
+    if (staged_f32_wins(m, n, k, transpose, b_f32, conv_elems, split)) return true;
+    *split = 1;
+    return dev->conv_bytes < conv_bytes && staged_f32_fits(m, n, k) && capturing(dev);
+}
+
 // One GEMM with f32 output on f32 operands: rounded to bf16 inside the kernel, or
 // converted into the scratch buffer first (staged_f32_wins, c_over_operand).
 // a_elems / b_elems: elements of A and B (0: already bf16).
@@ -1895,11 +1917,11 @@ static int matmul_common(t0g_device *dev, uint64_t a_f32, size_t a_elems, uint64
     std::lock_guard<std::mutex> lk(dev->mu);
     int rc = check_usable(dev);
     if (rc) return rc;
+    const size_t a_bytes = round256(a_elems * 2), b_bytes = round256(b_elems * 2);
     uint32_t split = 1;
     if (!c_over_operand(c, m, n, a_f32, a_elems) && !c_over_operand(c, m, n, b, b_elems) &&
-        staged_f32_wins(m, n, k, transpose, b_elems != 0, a_elems + b_elems, &split))
+        staged_f32(dev, m, n, k, transpose, b_elems != 0, a_elems + b_elems, a_bytes + b_bytes + 256, &split))
         return staged_f32_locked(dev, a_f32, b, b_elems != 0, c, m, n, k, transpose, split);
-    const size_t a_bytes = round256(a_elems * 2), b_bytes = round256(b_elems * 2);
     if ((rc = ensure_conv(dev, a_bytes + b_bytes + 256))) return rc;
     const uint64_t a16 = dev->conv, b16 = b_elems ? dev->conv + a_bytes : b;
     if ((rc = convert_pair_locked(dev, a_f32, a16, a_elems, b, b16, b_elems))) return rc;
@@ -2037,7 +2059,8 @@ static int matmul_cached(t0g_device *dev, uint64_t a_f32, size_t a_elems, uint64
     uint64_t w16 = 0;
     if (w_elems && (rc = bf16_cache_get_locked(dev, w_id, w, w_elems, &w16))) return rc;
     uint32_t split = 1;
-    if (!c_over_operand(c, m, n, a_f32, a_elems) && staged_f32_wins(m, n, k, transpose, false, a_elems, &split)) {
+    if (!c_over_operand(c, m, n, a_f32, a_elems) &&
+        staged_f32(dev, m, n, k, transpose, false, a_elems, round256(a_elems * 2) + 256, &split)) {
         if ((rc = staged_f32_locked(dev, a_f32, w16, false, c, m, n, k, transpose, split))) return rc;
         return ok();
     }

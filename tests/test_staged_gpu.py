@@ -268,3 +268,58 @@ def test_f32_output_over_an_operand(rt, m, k, n, call, over, shift):
         rt.clear_bf16_cache()
         for b in bufs:
             rt.free(b)
+
+
+# (m, k, n): K slices when the operands are rounded inside the GEMM (forward, data gradient),
+# and layers that are converted first
+@pytest.mark.parametrize("m,k,n", [(256, 1024, 512), (256, 512, 1024), (2048, 2048, 512)])
+def test_f32_calls_under_capture(m, k, n):
+    """A handle whose scratch buffers are not grown yet: a captured f32 call allocates nothing,
+    and every replay gives the eager result within the parity gate."""
+    from hip_rt import Graph, Stream
+    h = t0g.GpuRuntime.new(0)
+    s = Stream()
+    bufs, graphs = [], []
+    try:
+        rng = np.random.default_rng(m + k + n)
+        x = rng.uniform(-0.5, 0.5, (m, k)).astype(np.float32)
+        w = rng.uniform(-0.5, 0.5, (k, n)).astype(np.float32)
+        dy = rng.uniform(-0.5, 0.5, (m, n)).astype(np.float32)
+        xb, wb, dyb = (o.f32_to_bf16_rne(v) for v in (x, w, dy))
+        y_ref = o.gemm("NT", xb, np.ascontiguousarray(wb.T), m, n, k)
+        dx_ref = o.gemm("NT", dyb, wb, m, k, n)
+        ax, aw, ad = (h.upload(v) for v in (x, w, dy))
+        out = h.alloc(max(m * n, m * k) * 4)
+        bufs += [ax, aw, ad, out]
+        h.get_or_create_bf16(5, aw, k * n)
+        # loads the kernels; too small to be split or converted
+        for warm in (lambda: h.matmul_f32(ax, aw, out, 16, 64, 64), lambda: h.matmul_f32_cached(ax, aw, 6, out, 16, 64, 64),
+                     lambda: h.matmul_backward_data_f32(ad, aw, out, 16, 64, 64),
+                     lambda: h.matmul_backward_data_f32_cached(ad, aw, 6, out, 16, 64, 64)):
+            warm()
+        h.wait_idle()
+        h.set_stream(s.ptr)
+        for shape, ref, kk, call in (((m, n), y_ref, k, lambda: h.matmul_f32(ax, aw, out, m, k, n)),
+                                     ((m, n), y_ref, k, lambda: h.matmul_f32_cached(ax, aw, 5, out, m, k, n)),
+                                     ((m, k), dx_ref, n, lambda: h.matmul_backward_data_f32(ad, aw, out, m, k, n)),
+                                     ((m, k), dx_ref, n, lambda: h.matmul_backward_data_f32_cached(ad, aw, 5, out, m, k, n))):
+            before = t0g.device_alloc_count()
+            graphs.append(Graph(s, call))
+            assert t0g.device_alloc_count() == before
+            for _ in range(3):
+                h.memset(out, 0xFF, shape[0] * shape[1] * 4)
+                graphs[-1].launch(s)
+                s.synchronize()
+                ok, relf, maxabs, bound = o.parity(h.read(out, shape, np.float32), ref, kk)
+                assert ok, f"relF={relf:.3e} max|d|={maxabs:.3e} bound={bound:.3e}"
+                h.matmul_f32(ax, aw, out, 16, 64, 64)   # eager work between the replays
+                h.wait_idle()
+        h.set_stream(None)
+    finally:
+        for g in graphs:
+            g.destroy()
+        h.clear_bf16_cache()
+        for b in bufs:
+            h.free(b)
+        h.close()
+        s.destroy()
