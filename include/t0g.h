@@ -411,8 +411,7 @@ typedef struct t0g_compiled_kernel {
     uint32_t workgroup_size;    /* threads per workgroup along x (y = z = 1)  */
     uint32_t lds_size;          /* static LDS bytes                           */
     uint32_t kernarg_size;      /* bytes of kernargs[] to pass                */
-    uint32_t grid[3];           /* grid in threads for desc's problem (z > 1 only for unaligned
-                                 * operands and more than 2^22 tiles)             */
+    uint32_t grid[3];           /* grid in threads for desc's problem          */
     uint32_t splits;            /* fp32 planes written to C (1: C itself)      */
     uint8_t kernargs[160];      /* argument block for desc's problem           */
 } t0g_compiled_kernel;

@@ -205,18 +205,26 @@ __device__ __forceinline__ uint32_t xcd_range(uint32_t id, uint32_t total) {
     return x * q + min(x, r) + (id >> 3);
 }
 
-__device__ __forceinline__ GridPos grid_pos(const T0gGemmArgs& p, uint32_t tile) {
+// QUARTERS: a grid of very many tiles runs three quarters of them along y (T0G_QUARTERS_SHIFT).
+template <bool QUARTERS = false>
+__device__ __forceinline__ GridPos grid_pos(const T0gGemmArgs& p) {
     const uint32_t nblk = p.tiles_m * p.tiles_n;
-    uint32_t split = blockIdx.y;
+    uint32_t tile = blockIdx.x, split = blockIdx.y;
     const uint64_t total = (uint64_t)nblk * gridDim.y;
     if ((p.flags & T0G_FLAG_XCD_REMAP) && total <= 0xFFFFFFFFull) {
         const uint32_t l = xcd_range(split * nblk + tile, (uint32_t)total);
         split = l / nblk;
         tile = l - split * nblk;
+    } else if constexpr (QUARTERS) {
+        const uint32_t slices = p.flags >> T0G_QUARTERS_SHIFT;
+        if (slices != 0) {
+            const uint32_t part = (split >= slices) + (split >= 2 * slices) + (split >= 3 * slices);
+            tile += part * (nblk / 4);
+            split -= part * slices;
+        }
     }
     return GridPos{tile, split};
 }
-__device__ __forceinline__ GridPos grid_pos(const T0gGemmArgs& p) { return grid_pos(p, blockIdx.x); }
 
 template <int SM, int SN, bool OUT_BF16>
 __device__ __forceinline__ void store_tile(const T0gGemmArgs& p, const f32x16_t (&acc)[SM][SN], uint32_t row0,

@@ -296,9 +296,7 @@ __device__ __forceinline__ void gemm_tile_staged(const T0gGemmArgs& p) {
     __shared__ __attribute__((aligned(1024))) char smem[3 * STAGE];
 
     const uint32_t tid = threadIdx.x % NT;
-    const uint32_t linear = blockIdx.z * T0G_STAGED_TILES_X + blockIdx.x;
-    if (linear >= p.tiles_m * p.tiles_n) return;   // the last z's rest
-    const GridPos gp = grid_pos(p, linear);
+    const GridPos gp = grid_pos<true>(p);
     const uint32_t gm = p.group_m;
     const uint32_t per_group = gm * p.tiles_n;
     const uint32_t group = gp.tile / per_group;

@@ -132,9 +132,12 @@ typedef struct T0gConvertPairArgs {
     T0gConvertArgs a, b;
 } T0gConvertPairArgs;
 
-/* Tiles along grid x of the kernels that stage their operands through registers; further
- * ones go along z.  Their 512 threads would pass a grid's 2^32 threads along x from 2^23 tiles. */
-#define T0G_STAGED_TILES_X (1u << 22)
+/* The kernels that stage their operands through registers run 512 threads, so from 2^23
+ * tiles a grid would pass 2^32 threads along x.  It then holds a quarter of the tiles (a
+ * multiple of 4) along x and four times the K slices along y: flags >> T0G_QUARTERS_SHIFT is
+ * the number of slices (0 in all other launches), XCD_REMAP is not set, and y / slices is the
+ * quarter. */
+#define T0G_QUARTERS_SHIFT 16
 
 #define T0G_FLAG_XCD_REMAP 1u   /* remap workgroup ids so each XCD owns a contiguous tile (128x128, 64x64: (split, tile)) range */
 #define T0G_FLAG_C_VEC 2u       /* C base, row pitch and split-plane stride are 16-byte aligned */

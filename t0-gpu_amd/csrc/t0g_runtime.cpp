@@ -437,25 +437,6 @@ static int make_plan(const TileDef *tile, uint32_t transpose, bool out_bf16, Ope
     return T0G_OK;
 }
 
-// Workgroups of a plan's launch.  The staged kernels' tiles past T0G_STAGED_TILES_X
-// go along z: 1 x 600,000,000 x 3 has 9.4 Mi tiles of 64 columns, 4.8e9 threads.
-static void plan_grid(const GemmPlan &p, uint32_t grid[3]) {
-    const uint32_t tiles = p.tiles_m * p.tiles_n;
-    const bool along_z = !p.aligned && tiles > T0G_STAGED_TILES_X;
-    grid[0] = along_z ? T0G_STAGED_TILES_X : tiles;
-    grid[1] = p.splits;
-    grid[2] = along_z ? (tiles + T0G_STAGED_TILES_X - 1) / T0G_STAGED_TILES_X : 1;
-}
-
-// A launch takes less than 2^32 threads along x; the staged kernels keep the tile
-// count of 256-thread workgroups.  Refused here, before the launch: one that fails
-// poisons the handle.
-static int check_grid(const GemmPlan &p) {
-    if ((uint64_t)p.tiles_m * p.tiles_n * (p.aligned ? p.wg : 256u) > 0xFFFFFFFFull)
-        return fail(T0G_ERR_INVALID_ARG, "%u x %u tiles: the grid in threads exceeds 32 bits", p.tiles_m, p.tiles_n);
-    return T0G_OK;
-}
-
 // The staged kernels (operands the fast path cannot take) use 32-bit byte
 // offsets.
 static int check_extent(const char *what, uint64_t rows, uint64_t ld) {
@@ -511,6 +492,36 @@ static int ensure_sk_sync(t0g_device *dev) {
     return T0G_OK;
 }
 
+// Whether a staged kernel's launch is in four quarters of its tiles (T0G_QUARTERS_SHIFT):
+// 1 x 600,000,000 x 3 has 9.4 Mi tiles of 64 columns, 4.8e9 threads.
+static bool in_quarters(const GemmPlan &p) {
+    return !p.aligned && (uint64_t)p.tiles_m * p.tiles_n * p.wg > 0xFFFFFFFFull;
+}
+
+// A plan's launch: tile rows and columns (in quarters with a product in fours: tiles
+// past the output store nothing) and workgroups along x and y.
+struct PlanGrid {
+    uint32_t tiles_m, tiles_n, x, y;
+};
+static PlanGrid plan_grid(const GemmPlan &p) {
+    PlanGrid g = {p.tiles_m, p.tiles_n, p.tiles_m * p.tiles_n, p.splits};
+    if (in_quarters(p)) {
+        while (g.tiles_m * g.tiles_n % 4) ++(g.tiles_m > g.tiles_n ? g.tiles_m : g.tiles_n);
+        g.x = g.tiles_m * g.tiles_n / 4;
+        g.y *= 4;
+    }
+    return g;
+}
+
+// A launch takes less than 2^32 threads along x; the staged kernels keep the tile
+// count of 256-thread workgroups.  Refused here, before the launch: one that fails
+// poisons the handle.
+static int check_grid(const GemmPlan &p) {
+    if ((uint64_t)p.tiles_m * p.tiles_n * (p.aligned ? p.wg : 256u) > 0xFFFFFFFFull)
+        return fail(T0G_ERR_INVALID_ARG, "%u x %u tiles: the grid in threads exceeds 32 bits", p.tiles_m, p.tiles_n);
+    return T0G_OK;
+}
+
 // The GEMM kernel's argument block for a plan.  With splits > 1 and no
 // caller-owned planes (o.c_split_stride == 0) the kernel writes fp32 planes to
 // `ws` and *reduce is set: the reduce kernel then produces C.
@@ -528,10 +539,12 @@ static void fill_gemm_args(const GemmPlan &p, const GemmOperands &o, uint64_t ws
     args.lda = o.lda;
     args.ldb = o.ldb;
     args.k_per_split = p.k_per_split;
-    args.tiles_m = p.tiles_m;
-    args.tiles_n = p.tiles_n;
+    const PlanGrid grid = plan_grid(p);
+    args.tiles_m = grid.tiles_m;
+    args.tiles_n = grid.tiles_n;
     args.group_m = 8;
     args.flags = T0G_FLAG_XCD_REMAP | (allow_timeline && g_timeline.load() ? T0G_FLAG_TIMELINE : 0u);
+    if (in_quarters(p)) args.flags = (args.flags & ~T0G_FLAG_XCD_REMAP) | p.splits << T0G_QUARTERS_SHIFT;
     // Operands of 96 MB or more come from HBM as a rule (with the output and whatever
     // ran before, they do not stay in the 256 MiB Infinity Cache): the 256x256
     // kernels then prefetch into the L2.  Three sets of operands in turn, without
@@ -609,9 +622,8 @@ static int run_plan(t0g_device *dev, const GemmPlan &p, const GemmOperands &o, u
         dev->sk_stream = dev->stream;
         return launch(dev, f, sa.grid, 1, 1, p.wg, &sa, sizeof sa);
     }
-    uint32_t grid[3];
-    plan_grid(p, grid);
-    rc = launch(dev, f, grid[0], grid[1], grid[2], p.wg, &args, sizeof args);
+    const PlanGrid grid = plan_grid(p);
+    rc = launch(dev, f, grid.x, grid.y, 1, p.wg, &args, sizeof args);
     if (rc || !reduce) return rc;
 
     hipFunction_t fr = nullptr;
@@ -1536,8 +1548,10 @@ int t0g_gemm_compile(const t0g_gemm_desc *d, t0g_compiled_kernel *out) {
     out->workgroup_size = p.wg;
     out->lds_size = meta.group_segment_size;
     out->kernarg_size = (uint32_t)sizeof args;
-    plan_grid(p, out->grid);
-    out->grid[0] *= p.wg;
+    const PlanGrid grid = plan_grid(p);
+    out->grid[0] = grid.x * p.wg;
+    out->grid[1] = grid.y;
+    out->grid[2] = 1;
     out->splits = p.splits;
     memcpy(out->kernargs, &args, sizeof args);
     return ok();

@@ -453,20 +453,23 @@ def test_operand_size_limits(layout):
 
 def test_tile_counts_of_unaligned_products():
     """The kernels that stage their operands run 512 threads and take as many tiles as
-    256-thread workgroups would: 2^24 and no more, the ones past 2^22 along grid z."""
+    256-thread workgroups would: below 2^24, from 2^23 on in four quarters along grid y."""
     def compiled(n, k, preset=None):
         cfg = t0g.GemmConfig.preset(preset) if preset else None
         return t0g.gemm_compile(t0g.gemm_desc(1 << 20, 1 << 40, 1 << 44, 1, n, k, config=cfg))
 
-    for n, k, preset, tile in ((600_000_000, 3, None, 64), (1 << 28, 1, "gfx950_64x64_k64", 64),
-                               ((1 << 28) + 1, 1, "gfx950_64x64_k64", 64), ((1 << 30) - 64, 1, "gfx950_64x64_k64", 64),
+    for n, k, preset, tile in ((600_000_000, 3, None, 64), ((1 << 29) - 64, 1, "gfx950_64x64_k64", 64),
+                               (1 << 29, 1, "gfx950_64x64_k64", 64), ((1 << 30) - 64, 1, "gfx950_64x64_k64", 64),
                                ((1 << 31) - 200, 1, "gfx950_128x128_k64", 128)):
         ck = compiled(n, k, preset)
         assert ck.name.decode() == f"t0g_gemm_{tile}x{tile}_k64_nt_f32_u" and ck.workgroup_size == 512
-        tiles, per_z = -(-n // tile), ck.grid[0] // 512
-        assert ck.grid[0] % 512 == 0 and ck.grid[0] < 1 << 32 and ck.grid[1] == 1
-        assert per_z * (ck.grid[2] - 1) < tiles <= per_z * ck.grid[2]
-        assert ck.grid[2] == 1 if tiles <= 1 << 22 else per_z == 1 << 22
+        tiles, row = -(-n // tile), ck.grid[0] // 512
+        assert ck.grid[0] % 512 == 0 and ck.grid[0] < 1 << 32 and ck.grid[2] == 1
+        assert (row, ck.grid[1]) == ((tiles, 1) if tiles < 1 << 23 else ((tiles + 3) // 4, 4))
+    # with K slices: each quarter once per slice; 4097 x 2049 tiles, and three rows more are run
+    cfg = t0g.GemmConfig.preset("gfx950_64x64_k64")
+    ck = t0g.gemm_compile(t0g.gemm_desc(1 << 20, 1 << 40, 1 << 44, 4097 * 64, 2049 * 64, 130, config=cfg, split_k=2))
+    assert (ck.splits, ck.grid[0] // 512, ck.grid[1]) == (2, 4100 * 2049 // 4, 8)
     with pytest.raises(t0g.T0gError) as e:
         compiled(1 << 30, 1, "gfx950_64x64_k64")
     assert e.value.code == t0g.ERR_INVALID_ARG
