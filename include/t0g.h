@@ -473,6 +473,21 @@ T0G_API int t0g_matmul_f32_cached(t0g_device *dev, uint64_t x, uint64_t w, uint6
 T0G_API int t0g_matmul_backward_data_f32_cached(t0g_device *dev, uint64_t dy, uint64_t w, uint64_t w_id,
                                                 uint64_t dx, uint32_t m, uint32_t k, uint32_t n);
 
+/* The f32 calls above, for t0g_matmul_kernel_name. */
+typedef enum t0g_matmul_op {
+    T0G_MATMUL_FORWARD = 0,              /* t0g_matmul_f32                         */
+    T0G_MATMUL_BACKWARD_DATA = 1,        /* t0g_matmul_backward_data_f32           */
+    T0G_MATMUL_BACKWARD_WEIGHT = 2,      /* t0g_matmul_backward_weight_f32         */
+    T0G_MATMUL_FORWARD_CACHED = 3,       /* t0g_matmul_f32_cached                  */
+    T0G_MATMUL_BACKWARD_DATA_CACHED = 4, /* t0g_matmul_backward_data_f32_cached    */
+    T0G_MATMUL_WT_BF16 = 5               /* t0g_matmul_wt_bf16_f32                 */
+} t0g_matmul_op;
+/* Name of the GEMM kernel such a call runs and its number of K slices (diagnostics,
+ * no device needed; output over no operand): a suffix _ff or _fb says that the f32
+ * operands are rounded inside it, any other that they are converted first. */
+T0G_API int t0g_matmul_kernel_name(uint32_t op, uint32_t m, uint32_t k, uint32_t n, char *buf, size_t len,
+                                   uint32_t *splits);
+
 /* ---- GEMM autotuner and its on-disk cache ----------------------------------- *
  * GemmTuner (src/t0/auto_gemm.rs:28-417): benchmark the model's best candidate
  * configs on the GPU, keep the fastest, cache it in memory and as one JSON file

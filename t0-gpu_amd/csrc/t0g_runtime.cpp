@@ -1815,21 +1815,29 @@ static bool capturing(t0g_device *dev) {
     return T0G_HIP(hipStreamIsCapturing(dev->stream, &st)) != hipSuccess || st != hipStreamCaptureStatusNone;
 }
 
-// One GEMM with f32 output whose A (and, with b_f32, B) is f32, rounded to bf16
-// inside the kernel (64x64 tile, gemm_staged.h).  Without the memory for its planes
-// (a workspace that would grow under capture, or cannot grow) it runs unsplit.
+// The plan of a GEMM with f32 output whose A (and, with b_f32, B) is f32, rounded to
+// bf16 inside the kernel (64x64 tile, gemm_staged.h).
+static int staged_f32_plan(uint32_t m, uint32_t n, uint32_t k, uint32_t transpose, bool b_f32, uint32_t split,
+                           GemmPlan *p) {
+    int rc = make_plan(&kTiles[2], transpose, false, OperandPath::Staged, true, m, n, k, split, p);
+    if (rc) return rc;
+    p->symbol.replace(p->symbol.size() - 2, 2, b_f32 ? "_ff" : "_fb");
+    return T0G_OK;
+}
+
+// Run such a GEMM.  Without the memory for its planes (a workspace that
+// would grow under capture, or cannot grow) it runs unsplit.
 static int staged_f32_locked(t0g_device *dev, uint64_t a, uint64_t b, bool b_f32, uint64_t c, uint32_t m, uint32_t n,
                              uint32_t k, uint32_t transpose, uint32_t split) {
     GemmPlan p;
-    int rc = make_plan(&kTiles[2], transpose, false, OperandPath::Staged, true, m, n, k, split, &p);
+    int rc = staged_f32_plan(m, n, k, transpose, b_f32, split, &p);
     if (rc) return rc;
     if (p.splits > 1) {
         const size_t need = plan_workspace(p, m, n, dev->num_cus);
         rc = dev->ws_bytes < need && capturing(dev) ? (int)T0G_ERR_OUT_OF_MEMORY : ensure_workspace(dev, need);
         if (rc && rc != T0G_ERR_OUT_OF_MEMORY) return rc;
-        if (rc && (rc = make_plan(&kTiles[2], transpose, false, OperandPath::Staged, true, m, n, k, 1, &p))) return rc;
+        if (rc && (rc = staged_f32_plan(m, n, k, transpose, b_f32, 1, &p))) return rc;
     }
-    p.symbol.replace(p.symbol.size() - 2, 2, b_f32 ? "_ff" : "_fb");
     GemmOperands o;
     memset(&o, 0, sizeof o);
     o.a = a;
@@ -2102,6 +2110,40 @@ int t0g_matmul_f32_cached(t0g_device *dev, uint64_t x, uint64_t w, uint64_t w_id
 int t0g_matmul_backward_data_f32_cached(t0g_device *dev, uint64_t dy, uint64_t w, uint64_t w_id, uint64_t dx,
                                         uint32_t m, uint32_t k, uint32_t n) {
     return matmul_cached(dev, dy, (size_t)m * n, w, w_id, (size_t)k * n, dx, m, k, n, T0G_NT);
+}
+
+// The kernel and K slices of an f32 call whose output lies over no operand.
+int t0g_matmul_kernel_name(uint32_t op, uint32_t m, uint32_t k, uint32_t n, char *buf, size_t len, uint32_t *splits) {
+    if (!buf || !len) return fail(T0G_ERR_INVALID_ARG, "NULL argument");
+    if (op > T0G_MATMUL_WT_BF16) return fail(T0G_ERR_INVALID_ARG, "bad matmul op %u", op);
+    const bool data = op == T0G_MATMUL_BACKWARD_DATA || op == T0G_MATMUL_BACKWARD_DATA_CACHED;
+    const bool weight = op == T0G_MATMUL_BACKWARD_WEIGHT, forward = !data && !weight;
+    const bool b_f32 = op <= T0G_MATMUL_BACKWARD_WEIGHT;
+    const uint32_t t = weight ? T0G_TN : data || op == T0G_MATMUL_WT_BF16 ? T0G_NT : T0G_NN;
+    // rows, columns and contraction of the product
+    const uint32_t gm = weight ? k : m, gn = forward ? n : data ? k : n, gk = forward ? k : data ? n : m;
+    uint32_t split = 1;
+    GemmPlan p;
+    int rc;
+    if (staged_f32_wins(gm, gn, gk, t, b_f32, (uint64_t)gm * gk + (b_f32 ? (uint64_t)gk * gn : 0), &split)) {
+        rc = staged_f32_plan(gm, gn, gk, t, b_f32, split, &p);
+    } else {
+        t0g_gemm_desc d;
+        memset(&d, 0, sizeof d);
+        d.a = d.b = d.c = 4096;   // as aligned as the scratch buffer; not read here
+        d.m = gm;
+        d.n = gn;
+        d.k = gk;
+        d.transpose = t;
+        d.out_dtype = T0G_F32;
+        t0g_gemm_config cfg;
+        GemmOperands o;
+        rc = resolve_desc(&d, &cfg, &p, &o, true);
+    }
+    if (rc) return rc;
+    snprintf(buf, len, "%s", p.symbol.c_str());
+    if (splits) *splits = p.splits;
+    return ok();
 }
 
 }  // extern "C"

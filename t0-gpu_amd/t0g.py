@@ -40,6 +40,8 @@ NT, NN, TN, TT = 0, 1, 2, 3
 LAYOUTS = {"NT": NT, "NN": NN, "TN": TN, "TT": TT}
 EPI_STORE_F32, EPI_BIAS_ADD, EPI_BIAS_ADD_RELU = 0, 1, 2
 F32, BF16 = 0, 1
+(MATMUL_FORWARD, MATMUL_BACKWARD_DATA, MATMUL_BACKWARD_WEIGHT, MATMUL_FORWARD_CACHED, MATMUL_BACKWARD_DATA_CACHED,
+ MATMUL_WT_BF16) = range(6)
 STREAM_K = 0x80000000   # GemmConfig.split_k value selecting the stream-K schedule
 # tile_ir EpilogueOp (src/t0/tile_ir.rs:41-62): the fused epilogue chain
 OP_BIAS_ADD, OP_SCALE, OP_RELU, OP_SILU, OP_GELU, OP_ABS, OP_NEG, OP_CLAMP = range(1, 9)
@@ -283,6 +285,7 @@ _sig("t0g_bf16_cache_get", ctypes.c_int, _p, _u64, _u64, ctypes.c_size_t, ctypes
 _sig("t0g_bf16_cache_invalidate", ctypes.c_int, _p, _u64)
 _sig("t0g_bf16_cache_clear", ctypes.c_int, _p)
 _sig("t0g_bf16_cache_stats", ctypes.c_int, _p, ctypes.POINTER(_u64), ctypes.POINTER(_u64))
+_sig("t0g_matmul_kernel_name", ctypes.c_int, _u32, _u32, _u32, _u32, ctypes.c_char_p, ctypes.c_size_t, _u32p)
 _sig("t0g_matmul_f32_cached", ctypes.c_int, _p, _u64, _u64, _u64, _u64, _u32, _u32, _u32)
 _sig("t0g_matmul_backward_data_f32_cached", ctypes.c_int, _p, _u64, _u64, _u64, _u64, _u32, _u32, _u32)
 
@@ -504,6 +507,14 @@ def gemm_kernel_name(desc):
     buf = ctypes.create_string_buffer(128)
     _check(_lib.t0g_gemm_kernel_name(ctypes.byref(desc), buf, len(buf)))
     return buf.value.decode()
+
+
+def matmul_kernel_name(op, m, k, n):
+    """(kernel, K slices) of an f32 call (MATMUL_*) on a layer of m rows, k inputs and n outputs."""
+    buf = ctypes.create_string_buffer(128)
+    splits = ctypes.c_uint32()
+    _check(_lib.t0g_matmul_kernel_name(op, m, k, n, buf, len(buf), ctypes.byref(splits)))
+    return buf.value.decode(), splits.value
 
 
 def gemm_compile(desc):

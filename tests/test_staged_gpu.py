@@ -134,14 +134,22 @@ def _guarded_f32(rt, x):
 
 # (m, k, n) of the layer: the contraction is k forward, n for the data gradient, m for the
 # weight gradient; stage edges (63, 64, 65, 129 ...), rows of fewer than 4 values, ragged
-# tiles, sizes where K is split in the kernel (64 x 2048 x 64) and one that converts first
-# (300 x 1536 x 1544)
-LAYERS = [(32, 128, 128), (65, 63, 66), (64, 64, 64), (1, 65, 3), (3, 2, 130), (130, 129, 2), (127, 300, 191),
-          (64, 2048, 64), (5, 1000, 1001), (300, 1536, 1544)]
+# tiles.  With each layer the route of its six calls (forward, data and weight gradient, cached
+# forward and data gradient, bf16 weight): K slices of a GEMM that rounds the operands, 0 for
+# converted first, "?" where it is left to the rule.
+LAYERS = [(32, 128, 128, "111111"), (65, 63, 66, "111111"), (64, 64, 64, "111111"), (1, 65, 3, "111111"),
+          (3, 2, 130, "111111"), (130, 129, 2, "111111"), (127, 300, 191, "111111"), (64, 2048, 64, "811818"),
+          (5, 1000, 1001, "221???"), (300, 1536, 1544, "220???"), (2048, 2048, 2048, "000000")]
 
 
-@pytest.mark.parametrize("m,k,n", LAYERS)
-def test_f32_layers(rt, m, k, n):
+@pytest.mark.parametrize("m,k,n,routes", LAYERS)
+def test_f32_layers(rt, m, k, n, routes):
+    ops = (t0g.MATMUL_FORWARD, t0g.MATMUL_BACKWARD_DATA, t0g.MATMUL_BACKWARD_WEIGHT, t0g.MATMUL_FORWARD_CACHED,
+           t0g.MATMUL_BACKWARD_DATA_CACHED, t0g.MATMUL_WT_BF16)
+    for op, route in zip(ops, routes):
+        name, splits = t0g.matmul_kernel_name(op, m, k, n)
+        staged = name.endswith("_ff" if op <= t0g.MATMUL_BACKWARD_WEIGHT else "_fb")
+        assert route == "?" or route == (str(splits) if staged else "0"), (op, name, splits)
     rng = np.random.default_rng(m * 1009 + k * 31 + n)
     x = rng.uniform(-0.5, 0.5, (m, k)).astype(np.float32)
     w = rng.uniform(-0.5, 0.5, (k, n)).astype(np.float32)
