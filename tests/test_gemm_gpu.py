@@ -717,7 +717,7 @@ def _chain_case(m, n, k, layout, seed):
 @pytest.mark.parametrize("m,n,k", [(512, 512, 256), (300, 264, 192)])
 def test_epilogue_chains(rt, bufs, chain, preset, layout, m, n, k):
     """Every op of the chain in the store path of each kernel family (fast paths,
-    edge tiles, the element-wise path), f32 against the oracle and bf16 bit-exact
+    edge tiles, operands staged through registers), f32 against the oracle and bf16 bit-exact
     against RNE of the same kernel's f32 result."""
     a, b, a_st, b_st, bias = _chain_case(m, n, k, layout, 11)
     kw = dict(epilogue_ops=list(chain), epi_scale=-0.75, clamp=(-0.5, 1.25), bias=bufs.up(bias),
@@ -965,7 +965,7 @@ def test_gemm_group_equals_one_by_one(rt, bufs):
         ("NT", 128, 4096, 4096, t0g.BF16, {}, None),                            # 128x128 split 8
         ("TN", 512, 768, 1000, t0g.F32, {"epilogue_ops": ["bias", "silu"]}, None),
         ("NN", 4352, 4096, 1024, t0g.BF16, {"config": sk}, p256),               # stream-K asked for
-        ("TT", 300, 264, 1024, t0g.F32, {}, None),                              # element-wise rows
+        ("TT", 300, 264, 1024, t0g.F32, {}, None),                              # unaligned rows   
     ]
     bias = bufs.up(np.linspace(-1, 1, 768, dtype=np.float32))
     descs, singles, outs = [], [], []

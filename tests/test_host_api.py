@@ -281,7 +281,7 @@ def test_gemm_plan_selection_host_only():
     d = t0g.gemm_desc(0x10000, 0x20000, 0x30000, 4096, 4096, 4096, transpose="NN", out_dtype=t0g.BF16)
     assert t0g.gemm_kernel_name(d) == "t0g_gemm_256x256_k64_nn_bf16"
     assert t0g.gemm_workspace_size(d) == 0
-    d = t0g.gemm_desc(0x10000, 0x20000, 0x30000, 33, 50, 100)          # K % 8 != 0: element-wise loads
+    d = t0g.gemm_desc(0x10000, 0x20000, 0x30000, 33, 50, 100)          # K % 8 != 0: staged through registers
     assert t0g.gemm_kernel_name(d).endswith("_u")
     d = t0g.gemm_desc(0x10000, 0x20000, 0x30000, 256, 256, 32768)
     assert "_nt_f32" in t0g.gemm_kernel_name(d)            # split-K: f32 partial planes
@@ -418,8 +418,8 @@ def test_operand_size_limits(layout):
     """Operands below 2^30 elements take the fast kernels; larger aligned ones the wide
     256x256 kernels (_x: descriptors rebased per tile or K stage), whatever the config
     asked for, as long as the leading dimension stays below 2^22 (K-contiguous) or
-    2^24 - 256 (M/N-contiguous) elements; the rest goes element-wise (_u, 32-bit element
-    offsets), where 2^31 elements or more are refused with an error."""
+    2^24 - 256 (M/N-contiguous) elements; the rest is staged through registers (_u, 32-bit
+    byte offsets), where 2^31 elements or more are refused with an error."""
     k, n = 16384, 256
     a, b = 1 << 12, 1 << 40   # 16-byte aligned device addresses (not dereferenced here)
 
@@ -435,18 +435,18 @@ def test_operand_size_limits(layout):
     assert name((1 << 31) // k, config=c128.copy(split_k=2)) == f"t0g_gemm_256x256_k64_{layout.lower()}_f32_x"
     sk = t0g.GemmConfig.preset("gfx950_256x256_k64").copy(split_k=t0g.STREAM_K)
     assert name((1 << 31) // k, config=sk).endswith("_bf16_x")                     # no wide stream-K kernel
-    # unaligned A: element-wise, refused once A spans 2^31 elements
+    # unaligned A: staged through registers, refused once A spans 2^31 elements
     assert name((1 << 31) // k - 8, a=a + 2).endswith("_u")
     with pytest.raises(t0g.T0gError) as e:
         name((1 << 31) // k, a=a + 2)
     assert e.value.code == t0g.ERR_INVALID_ARG
-    # leading dimensions past the wide kernels' offset range: element-wise
+    # leading dimensions past the wide kernels' offset range: staged
     a_k = layout in ("NT", "NN")
     big_ld = (1 << 22) if a_k else (1 << 24)
     m = 1 << 12 if a_k else big_ld - 512      # A of about 2^34 (K-contiguous) or 2^31 (M/N-contiguous) elements
     kk = k if a_k else 128
     assert name(m, k=kk, lda=big_ld - 512).endswith("_x")
-    with pytest.raises(t0g.T0gError) as e:    # past the bound: element-wise, which cannot take 2^31 elements
+    with pytest.raises(t0g.T0gError) as e:    # past the bound: staged, which cannot take 2^31 elements
         name(m, k=kk, lda=big_ld)
     assert e.value.code == t0g.ERR_INVALID_ARG
 

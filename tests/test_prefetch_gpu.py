@@ -22,12 +22,12 @@ def rt():
 
 def _prefetches(desc):
     flags = struct.unpack_from("<I", t0g.gemm_compile(desc).args(), 40 + 11 * 4)[0]
-    return bool(flags & 32)   # T0G_FLAG_PREFETCH
+    return bool(flags & 32)   # T0G_FLAG_PREFETCH: the prefetching loop, if the K range is whole stages
 
 
 @pytest.mark.parametrize("layout", ["NT", "NN", "TN", "TT"])
 @pytest.mark.parametrize("m,n,k,split", [(264, 12032, 4096, 1), (520, 11776, 4096, 1), (1032, 4608, 9088, 1),
-                                         (2056, 10240, 4104, 1), (264, 5888, 8192, 4)])
+                                         (2056, 10240, 4096, 1), (2056, 10240, 4104, 1), (264, 5888, 8192, 4)])
 def test_prefetch_changes_no_bit(rt, layout, m, n, k, split):
     assert 2 * k * (m + n) >= 96e6 and 2 * k * (m + n // 2) < 96e6
     rng = np.random.default_rng(m + n + k)

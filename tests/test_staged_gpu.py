@@ -107,6 +107,49 @@ def test_more_tiles_than_a_grid_row(rt):
 
 
 @pytest.mark.parametrize("preset", ["gfx950_64x64_k64", "gfx950_128x128_k64"])
+@pytest.mark.parametrize("layout,rows,ld,k", [("NT", 32764, 65537, 200), ("TN", 131, 16392001, 131)])
+def test_offsets_to_the_last_bit(rt, layout, preset, rows, ld, k):
+    """An unaligned operand of about 2^31 - 2^17 elements, so that 32-bit byte offsets run up to
+    their last values: whole stages and the edge stage, a K-contiguous B and an M-contiguous A.  All of it
+    is NaN but the rows (columns) of C that are looked at, at both ends of the operand."""
+    assert (1 << 31) - (1 << 18) < rows * ld < 1 << 31
+    other, size = 3, rows if layout == "NT" else ld          # the operand's M/N extent
+    pieces = ((0, 70), (size - 300, 300))                    # where it holds values
+    rng = np.random.default_rng(rows)
+    few = o.f32_to_bf16_rne(rng.uniform(-0.5, 0.5, (other, k)).astype(np.float32))
+    many = {s: o.f32_to_bf16_rne(rng.uniform(-0.5, 0.5, (c, k)).astype(np.float32)) for s, c in pieces}
+    big = rt.alloc(rows * ld * 2)
+    df = rt.upload(few if layout == "NT" else np.ascontiguousarray(few.T))
+    dc = rt.alloc(other * size * 4)
+    try:
+        rt.memset(big, 0xFF, rows * ld * 2)
+        for s, v in many.items():
+            if layout == "NT":
+                for r in range(len(v)):
+                    rt.write(big + (s + r) * ld * 2, v[r])
+            else:
+                for r in range(k):
+                    rt.write(big + (r * ld + s) * 2, np.ascontiguousarray(v[:, r]))
+        m, n, a, b = (other, size, df, big) if layout == "NT" else (size, other, big, df)
+        d = t0g.gemm_desc(a, b, dc, m, n, k, transpose=layout, lda=k if layout == "NT" else ld,
+                          ldb=ld if layout == "NT" else other, split_k=1, config=t0g.GemmConfig.preset(preset))
+        assert t0g.gemm_kernel_name(d).endswith("_u")
+        rt.memset(dc, 0, other * size * 4)
+        rt.gemm_desc(d)
+        rt.wait_idle()
+        c = rt.read(dc, (m, n), np.float32)
+        c = c.T if layout == "NT" else c                     # [operand row][other]
+        for s, v in many.items():
+            ref = o.gemm("NT", v, few, len(v), other, k)
+            ok, relf, maxabs, bound = o.parity(np.ascontiguousarray(c[s:s + len(v)]), ref, k)
+            assert ok, f"at {s}: relF={relf:.3e} max|d|={maxabs:.3e} bound={bound:.3e}"
+        assert np.all(np.isnan(c[70:size - 300]))
+    finally:
+        for x in (big, df, dc):
+            rt.free(x)
+
+
+@pytest.mark.parametrize("preset", ["gfx950_64x64_k64", "gfx950_128x128_k64"])
 @pytest.mark.parametrize("layout", ["NT", "NN"])
 @pytest.mark.parametrize("k", [5, 64, 333])
 def test_dispatch_of_no_columns(rt, layout, preset, k):

@@ -2,7 +2,7 @@
 
 Each case draws a layout (NT/NN/TN/TT), M, N and K, a config (auto_select's or one of
 the three tiles), a split-K count, padded leading dimensions (some of them not a
-multiple of 8, which routes the operands to the element-wise kernels) and the
+multiple of 8, which routes the operands to the kernels that stage them) and the
 output type; every third case also an epilogue chain of one to four ops with
 random bias, scale and clamp bounds (checked against the oracle's restatement of
 the chain).  Even cases draw A and B from the reference's LCG (one-sided, U[-0.5, 0]); odd
@@ -73,7 +73,7 @@ def _stored(logical, pad, rng):
 # grid stays at one workgroup per CU and slices of 24 stages or more reach the deep ring's
 # K-split kernels (_ds, and _dsr where two slices are summed in the kernel); the short-K
 # sweep above never gets there.  Padding of 13 elements still sends some cases to the
-# element-wise kernels.  16 committed; 120 pass with T0G_SWEEP_LONG_CASES=120.
+# _u kernels.  16 committed; 120 pass with T0G_SWEEP_LONG_CASES=120.
 N_LONG = int(os.environ.get("T0G_SWEEP_LONG_CASES", "16"))
 
 
