@@ -545,15 +545,22 @@ static void fill_gemm_args(const GemmPlan &p, const GemmOperands &o, uint64_t ws
     args.group_m = 8;
     args.flags = T0G_FLAG_XCD_REMAP | (allow_timeline && g_timeline.load() ? T0G_FLAG_TIMELINE : 0u);
     if (in_quarters(p)) args.flags = (args.flags & ~T0G_FLAG_XCD_REMAP) | p.splits << T0G_QUARTERS_SHIFT;
-    // Operands of 96 MB or more come from HBM as a rule (with the output and whatever
-    // ran before, they do not stay in the 256 MiB Infinity Cache): the 256x256
-    // kernels then prefetch into the L2.  Three sets of operands in turn, without
-    // and with it: 1024 x 11008 x 4096 NN (99 MB) 88.0 / 81.5 us, NT 93.7 / 80.8, 2048 x
-    // 11008 x 4096 NT 186.9 / 168.1, 8192^3 NN 776.8 / 754.6, NT 792.6 / 749.6, 5120^3
-    // 221.0 / 216.8; below, what a prefetch costs shows: 4096^3 (67 MB) NN 95.7 / 98.0,
-    // 4096 x 5120 x 4096 (75 MB) 160.8 / 164.7, 11008 x 4096 x 1024 TN (31 MB) 83.4 / 86.0.
-    // One shape above it lost, 6144^3 NN 381.2 / 387.0 (NT 380.3 / 370.7).
-    if (p.tile->bm == 256 && 2.0 * o.k * ((double)o.m + o.n) >= 96e6) args.flags |= T0G_FLAG_PREFETCH;
+    // The 256x256 kernels prefetch into the L2 from 96 MB of operands on: those come from
+    // HBM as a rule (with the output and whatever ran before, they do not stay in the 256 MiB
+    // Infinity Cache).  Without and with it, three sets of operands in turn: 1024 x 11008
+    // x 4096 NN (99 MB) 93.1 / 83.0 us, NT 93.1 / 81.7, 2048 x 11008 x 4096 NT 190.3 / 170.2,
+    // 8192^3 NN 783 / 759, NT 792 / 753, 5120^3 NN 231 / 214; 84 MB, which three sets hold in
+    // that cache, 1024 x 9216 x 4096 75.8 / 77.4 and 4608^3 185 / 190, 92 MB either way.  A call
+    // that finds its operands cached pays 2 to 5 % for the touches (8192^3 NT 700 / 733, one
+    // set), which is what the line weighs.  Beyond two rounds of workgroups only tile rows that
+    // are a power of two gain (16 x 36 tiles 290 / 279, 32 x 26 388 / 376, 64 x 16 320 /
+    // 312).  With others HBM costs little anyway (6144^3, 24 x 24 tiles, 376 us cached, 382
+    // not; the XCDs then presumably stream a panel at different times) and the touches more: 382 /
+    // 388, 28 x 28 364 / 370, 40 x 26 460 / 473, 96 x 11 248 / 259, 20 x 43 376 / 382.
+    const uint64_t wgs = (uint64_t)p.tiles_m * p.tiles_n * p.splits;
+    if (p.tile->bm == 256 && 2.0 * o.k * ((double)o.m + o.n) >= 96e6 &&
+        (wgs <= 2 * kNumCUs || (p.tiles_m & (p.tiles_m - 1)) == 0))
+        args.flags |= T0G_FLAG_PREFETCH;
     const bool reduce = p.splits > 1 && o.c_split_stride == 0 && !p.fused;
     if (reduce) {
         args.c = ws;

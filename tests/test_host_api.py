@@ -451,6 +451,21 @@ def test_operand_size_limits(layout):
     assert e.value.code == t0g.ERR_INVALID_ARG
 
 
+def test_prefetch_rule():
+    """The 256x256 kernels prefetch from 96 MB of operands on, beyond two rounds of tiles only where
+    the tile rows are a power of two."""
+    def flag(m, n, k, layout="NN", **kw):
+        d = t0g.gemm_desc(1 << 12, 1 << 40, 1 << 41, m, n, k, transpose=layout, out_dtype=t0g.BF16,
+                          config=t0g.GemmConfig.preset("gfx950_256x256_k64"), split_k=1, **kw)
+        return bool(struct.unpack_from("<I", t0g.gemm_compile(d).args(), 40 + 11 * 4)[0] & 32)
+
+    assert not flag(4096, 4096, 4096) and not flag(1024, 9216, 4096)           # below the line
+    assert flag(1024, 11008, 4096) and flag(5120, 5120, 5120)                   # 172 and 400 tiles
+    for layout in ("NN", "NT", "TN", "TT"):
+        assert flag(8192, 8192, 8192, layout) and flag(4096, 11008, 4096, layout)   # 32 and 16 tile rows
+        assert not flag(6144, 6144, 6144, layout) and not flag(11008, 4096, 4096, layout)   # 24 and 43
+
+
 def test_tile_counts_of_unaligned_products():
     """The kernels that stage their operands run 512 threads and take as many tiles as
     256-thread workgroups would: below 2^24, from 2^23 on in four quarters along grid y."""
