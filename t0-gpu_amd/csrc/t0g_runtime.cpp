@@ -1803,8 +1803,8 @@ static int convert_locked(t0g_device *dev, uint64_t src, uint64_t dst, uint64_t 
     return launch(dev, f, a.grid_blocks, 1, 1, 256, &a, sizeof a);
 }
 
-// Two operands in one launch: a launch of its own costs the smaller one 3 to 4 us,
-// its conversion beside the larger one's next to nothing.
+// Two operands in one launch: a launch of its own costs the smaller one 2 us back to
+// back, its conversion beside the larger one's next to nothing.
 static int convert_pair_locked(t0g_device *dev, uint64_t src0, uint64_t dst0, uint64_t n0, uint64_t src1,
                                uint64_t dst1, uint64_t n1) {
     if (n0 == 0) return convert_locked(dev, src1, dst1, n1);
@@ -1871,14 +1871,17 @@ static bool staged_f32_fits(uint32_t m, uint32_t n, uint32_t k) {
 // the conversion's launch and pass weigh more than a slower K loop: small and
 // ordinary layers.  Converting first against inside, one box: 32x128x128 forward
 // 7.6 / 4.7 us, 1024^3 forward 14.2 / 12.1, its data gradient with a cached weight
-// 12.1 / 9.4, 512x3072x768 data gradient 18.2 / 15.0 (split 2); but 2048x2048x512
-// forward 15.6 / 20.9, 768x3072x512 weight gradient 12.5 / 15.5.
+// 12.1 / 9.4, 512x3072x768 data gradient 18.2 / 15.0 (split 4); but 2048x2048x512
+// forward 15.6 / 20.9, 768x3072x512 weight gradient 12.5 / 15.5.  Of 2670 calls of 500
+// random layers (to 2048 rows, 4096 inputs and outputs) that it takes, 93 % gain more
+// than 3 % and 2.5 % lose as much, where its estimate is further off than that.
 static bool staged_f32_wins(uint32_t m, uint32_t n, uint32_t k, uint32_t transpose, bool b_f32, uint64_t conv_elems,
                             uint32_t *split) {
     if (!staged_f32_fits(m, n, k)) return false;
     t0g_gemm_config cfg;
     select_config(m, k, n, &cfg, false);
     double conv = 3.0 + 6.0 * (double)conv_elems / 4.5e6;
+    const double pass = conv;   // launch and bytes
     const bool aligned = operand_path(0, 0, m, n, k, a_k_major(transpose) ? k : m, b_k_major(transpose) ? k : n,
                                       transpose) != OperandPath::Staged;
     // unaligned operands are staged as bf16 then, at about 0.7 of the fast kernels' rate
@@ -1889,7 +1892,12 @@ static bool staged_f32_wins(uint32_t m, uint32_t n, uint32_t k, uint32_t transpo
     bool wins = false;
     for (uint32_t sk = 1; sk <= 8; sk *= 2) {
         if (sk > 1 && k < sk * 4 * kTileK) break;
-        const double per_cu = tiles * sk / kNumCUs, steps = ceil((double)k / sk / kTileK);
+        double per_cu = tiles * sk / kNumCUs;
+        const double steps = ceil((double)k / sk / kTileK);
+        // two workgroups share a CU, a third waits: 1216x1920x144 weight gradient (570 tiles)
+        // 9.0 / 13.5 us; with long slices the CUs that hold two set the time: 191x3136x3712,
+        // 294 workgroups of 29 steps, 19.4 / 26.7 us
+        if (sk == 1 ? per_cu > 2.0 : per_cu > 1.0 && steps >= 20.0) per_cu = ceil(per_cu);
         double t = 3.5 + (per_cu > 1.0 ? per_cu : 1.0) * (steps * stage + 1.0);
         if (sk > 1) t += 2.5 + (double)sk * m * n * 4.0 / 4.5e6 + 0.25 * sk;   // as model_time_us
         if (t < best) {
@@ -1898,6 +1906,14 @@ static bool staged_f32_wins(uint32_t m, uint32_t n, uint32_t k, uint32_t transpo
             *split = sk;
         }
     }
+    // The DMA waves of an unsplit 64x64 bf16 GEMM take a step in 0.12 us, half the model's time:
+    // with one f32 operand and no split, converting wins from about 12 steps on.  64 rows x
+    // 1024 -> 4096 with a bf16 weight 8.1 / 9.5 us, 16 steps in 2 tiles 7.4 / 8.5; 8 steps
+    // gain 12 % inside, 16 in 4 slices 10 %.
+    const double all_steps = ceil((double)k / kTileK);
+    if (wins && *split == 1 && !b_f32 && aligned && cfg.tile_m == 64 && cfg_split(&cfg) == 1 && tiles <= kNumCUs &&
+        all_steps < kKsplitMinStages && best > 1.03 * (pass + 3.75 + 0.12 * all_steps))
+        wins = false;
     return wins;
 }
 

@@ -182,7 +182,8 @@ def _guarded_f32(rt, x):
 # converted first, "?" where it is left to the rule.
 LAYERS = [(32, 128, 128, "111111"), (65, 63, 66, "111111"), (64, 64, 64, "111111"), (1, 65, 3, "111111"),
           (3, 2, 130, "111111"), (130, 129, 2, "111111"), (127, 300, 191, "111111"), (64, 2048, 64, "811818"),
-          (5, 1000, 1001, "221???"), (300, 1536, 1544, "220???"), (2048, 2048, 2048, "000000")]
+          (5, 1000, 1001, "221???"), (300, 1536, 1544, "220???"), (2048, 2048, 2048, "000000"),
+          (64, 1024, 4096, "480080"), (144, 1216, 1920, "??00??")]
 
 
 @pytest.mark.parametrize("m,k,n,routes", LAYERS)
