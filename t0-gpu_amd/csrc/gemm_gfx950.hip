@@ -84,11 +84,6 @@ __device__ __forceinline__ void tl_mark(const T0gGemmArgs& p, int ev) {
 #endif
 }
 
-__device__ __forceinline__ u32x4_t pack8(const uint16_t e[8]) {
-    return u32x4_t{(uint32_t)e[0] | ((uint32_t)e[1] << 16), (uint32_t)e[2] | ((uint32_t)e[3] << 16),
-                   (uint32_t)e[4] | ((uint32_t)e[5] << 16), (uint32_t)e[6] | ((uint32_t)e[7] << 16)};
-}
-
 // ---------------------------------------------------------------------------
 // Epilogue: acc -> epilogue chain -> f32 or bf16 (round to nearest even),
 // masked to the M x N output.  32x32 MFMA result layout: lane

@@ -94,8 +94,7 @@ struct StagedOperand {
         row0 = first;
         rows = R;
         const uint32_t outside = R >= kVals ? R - kVals : 0;   // columns read by pieces wholly past the operand
-        last_col = min(row0 + ROWS - kVals, (R - 1) & ~(kVals - 1));
-        if (row0 + ROWS > R && last_col < outside) last_col = outside;
+        last_col = min(row0 + ROWS - kVals, (R - 1) & ~(kVals - 1));   // not below `outside` where that is read
         slot = tid * kSlot;
 #pragma unroll
         for (int i = 0; i < kPieces; ++i) {
