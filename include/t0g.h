@@ -318,7 +318,9 @@ T0G_API int t0g_code_object_kernel_meta(const void *code_object, size_t size, co
  * kernel's argument size is read from the code object's metadata, and every
  * dispatch of it must pass exactly that many kernarg bytes (T0G_ERR_INVALID_ARG
  * otherwise, before anything reaches the GPU; this library's GEMM kernels take
- * 104).  A workgroup larger than the kernel was built for is refused here.
+ * 104).  A workgroup larger than the kernel was built for is refused here.  This
+ * library's 64x64 and 128x128 kernels built for 512 threads may be loaded with 256,
+ * their config's wg_size: each dispatch adds the four waves that fetch operands.
  * lds_size is the kernel's total LDS, as in KernelLoadConfig: the part beyond
  * the kernel's static LDS is requested as dynamic LDS at launch. */
 T0G_API int t0g_kernel_load(t0g_device *dev, const void *code_object, size_t size,
