@@ -35,7 +35,8 @@ def _embed(rt, stored, pad, lead):
 
 # (m, n, k): stage edges with 2 (128x128) and 4 (64x64) stages in flight, tile edges, tiny rows
 SHAPES = [(65, 63, 63), (64, 64, 65), (63, 129, 64 * 4 + 1), (127, 66, 64 * 5 - 1), (129, 127, 64 * 8 + 7),
-          (130, 70, 64 * 9), (33, 257, 7), (257, 31, 8), (5, 90, 321), (90, 3, 130), (1, 1, 200), (2, 67, 5)]
+          (130, 70, 64 * 9), (33, 257, 7), (257, 31, 8), (5, 90, 321), (90, 3, 130), (1, 1, 200), (2, 67, 5),
+          (70, 130, 1), (129, 65, 3), (1, 66, 5), (3, 2, 2), (1, 1, 1)]
 
 
 @pytest.mark.parametrize("layout", ["NT", "NN", "TN", "TT"])
@@ -181,7 +182,7 @@ def _guarded_f32(rt, x):
 # forward and data gradient, bf16 weight): K slices of a GEMM that rounds the operands, 0 for
 # converted first, "?" where it is left to the rule.
 LAYERS = [(32, 128, 128, "111111"), (65, 63, 66, "111111"), (64, 64, 64, "111111"), (1, 65, 3, "111111"),
-          (3, 2, 130, "111111"), (130, 129, 2, "111111"), (127, 300, 191, "111111"), (64, 2048, 64, "811818"),
+          (3, 2, 130, "111111"), (130, 129, 2, "111111"), (66, 1, 3, "111111"), (1, 2, 1, "111111"), (127, 300, 191, "111111"), (64, 2048, 64, "811818"),
           (5, 1000, 1001, "221???"), (300, 1536, 1544, "220???"), (2048, 2048, 2048, "000000"),
           (64, 1024, 4096, "480080"), (144, 1216, 1920, "??00??")]
 
